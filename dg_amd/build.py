@@ -35,6 +35,7 @@ SOURCES = [
     ("capi.cc", "hip-host", []),
     ("rhs.hip", "hipcc", []),
     ("stage.hip", "hipcc", []),
+    ("step1d.hip", "hipcc", []),
     ("batch.hip", "hipcc", []),
     ("mlp.hip", "hipcc", []),
     ("limiter.hip", "hipcc", ["-ffp-contract=off"]),

@@ -109,16 +109,17 @@ dgx_status fail(int code, const std::string& msg) {
 
 
 // Checks that the mesh is a Cartesian grid whose faces follow the structured
-// pattern the tile kernel assumes (element e = ey*nx + ex; side 0 is the
+// pattern the grid kernels assume (element e = ey*nx + ex; side 0 is the
 // left/lower element, or the boundary element of a boundary face; closures
 // and periodic partners as built by build_tables; normals along the axes)
 // and gathers each face's normal and Jacobians into grid order.  Any
-// mismatch leaves the general path.
+// mismatch leaves the general path.  True when its sides are whole tiles
+// too; out.grid when only the pattern holds.
 bool cartesian_layout(const Tables& t, Cart& out) {
   Cart c;
   const int D = t.D, nx = t.nx, ny = (D == 2) ? t.ny : 1;
   if (nx * ny != t.N_E) return false;
-  if (!stage_tiles(D, nx, ny, &c.tx, &c.ty)) return false;
+  const bool whole_tiles = stage_tiles(D, nx, ny, &c.tx, &c.ty);
   c.nx = nx;
   c.ny = ny;
   for (int k = 0; k < 4; ++k) c.bc[k] = t.bc[k];
@@ -168,9 +169,10 @@ bool cartesian_layout(const Tables& t, Cart& out) {
     if (!v) return false;
   for (char v : seen_y)
     if (!v) return false;
-  c.on = true;
+  c.grid = true;
+  c.on = whole_tiles;
   out = std::move(c);
-  return true;
+  return out.on;
 }
 
 }  // namespace
@@ -351,7 +353,7 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
             upload(s, &s.t.Minv, t.Minv.data(), uniform_minv ? (size_t)Ns * Ns : t.Minv.size()) &&
             upload(s, &s.t.neighbors, t.neighbors.data(), t.neighbors.size()) &&
             upload(s, &s.t.weight, t.weight.data(), t.weight.size());
-  if (ok && s.cart.on)
+  if (ok && s.cart.grid)
     ok = upload(s, &s.t.face_geo_x, s.cart.gx.data(), s.cart.gx.size()) &&
          upload(s, &s.t.face_geo_y, s.cart.gy.data(), s.cart.gy.size());
   if (ok && D == 1)
@@ -394,10 +396,17 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
        alloc(s, &s.work, S) && alloc(s, &s.work2, S) && alloc(s, &s.Uavg, (size_t)NE * s.NF) &&
        alloc(s, &s.sensors, (size_t)NE) && alloc(s, &s.sens_tgt, (size_t)2 * NE) &&
        alloc(s, &s.sens_act, (size_t)3 * NE) && alloc(s, &s.flag, 4) && alloc(s, &s.sens_changed, kRelaxBatch) && alloc(s, &s.flag_list, (size_t)NE) &&
-       alloc(s, &s.dscratch, 8) && alloc(s, &s.time_state, 4) &&
+       alloc(s, &s.dscratch, 8) && alloc(s, &s.time_state, 8) &&
        alloc(s, &s.cons_partial, conservation_scratch_doubles()) &&
        alloc(s, &s.dt_partial, ((size_t)NE * Ns + 255) / 256 + 1) &&
        ((!s.cart.on && D != 1) || alloc(s, &s.Ustar2, S));
+  // the 1D whole-step kernel: one shared mass matrix (to J), both ends
+  // periodic or neither
+  if (ok && D == 1 && s.cart.grid && uniform_minv &&
+      (s.cart.bc[0] == BC_PERIODIC) == (s.cart.bc[1] == BC_PERIODIC)) {
+    s.part1d_len = 1 + std::max(step1d_shape(s.P, NE, false).blocks, step1d_shape(s.P, NE, true).blocks);
+    ok = alloc(s, &s.part1d, (size_t)2 * s.part1d_len + 2);
+  }
   if (ok) ok = hip_ok(hipMemset(s.sensors, 0, sizeof(int) * NE), "hipMemset");
   if (!ok) {
     free_solver(s);
@@ -542,8 +551,31 @@ static dgx_status timed_hr_oop(Solver& s, const double* In, double* Out, hipStre
   return hip_ok(launch_limit_hr_oop(s, In, Out, st), "HR limiter") ? DGX_OK : DGX_EDEVICE;
 }
 
+// one 1D step In -> Out in one launch, with Dt at dt
+static dgx_status step1d_fixed(Solver& s, const double* In, double* Out, const double* dt, int limiter,
+                               hipStream_t st) {
+  KernelTimer kt(s, 4, st);
+  Step1DRun run;
+  run.In = In;
+  run.Out = Out;
+  run.limited = limiter == 1;
+  run.dt_fixed = dt;
+  return hip_ok(launch_step1d(s, run, st), "1D step kernel") ? DGX_OK : DGX_EDEVICE;
+}
+
+static dgx_status copy_state(const Solver& s, double* dst, const double* src, hipStream_t st) {
+  if (dst == src) return DGX_OK;
+  return hip_ok(hipMemcpyAsync(dst, src, sizeof(double) * s.state_size(), hipMemcpyDeviceToDevice, st), "copy")
+             ? DGX_OK
+             : DGX_EDEVICE;
+}
+
 static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, hipStream_t st) {
   dgx_status r;
+  if (s.step1d(limiter)) {
+    if ((r = step1d_fixed(s, U, s.Ustar, dt, limiter, st)) != DGX_OK) return r;
+    return copy_state(s, U, s.Ustar, st);
+  }
   if (DGX_RK_HR2D && limiter == 1 && ((s.tiled() && s.hr2d) || s.D == 1)) {
     // One-launch HR limiter (out of place; 2D tiles, or 1D): every stage
     // writes Ustar, the limiter takes Ustar to Ustar2 (the next stage's input)
@@ -669,6 +701,71 @@ static dgx_status integrate_cfl_device(Solver& s, double* U, double cfl, int nst
   return DGX_OK;
 }
 
+// The same for the 1D whole-step kernel: the initial limit and the first
+// maxima of |u|+a in one launch, then one launch per step that takes its Dt
+// from the maxima the launch before it left (k_step1d).  The state moves
+// between U and Ustar; steps queued after the end leave both as they are, so
+// the number of steps taken says where it is.
+static dgx_status integrate_cfl_step1d(Solver& s, double* U, double cfl, int nsteps, double tf, int limiter,
+                                       int* n_out_steps, double* T_out, hipStream_t st) {
+  const int nblk = step1d_shape(s.P, s.N_E, limiter == 1).blocks;
+  double* part[2] = {s.part1d, s.part1d + s.part1d_len};
+  double* dev[2] = {s.dscratch + 4, s.dscratch + 6};
+  int* state[2] = {s.time_state, s.time_state + 4};
+  double* buf[2] = {U, s.Ustar};
+  if (limiter == 1) std::swap(buf[0], buf[1]);  // the initial limit goes from U to Ustar
+  {
+    KernelTimer kt(s, 2, st);
+    Step1DRun run;
+    run.In = U;
+    run.Out = limiter == 1 ? s.Ustar : nullptr;
+    run.limited = limiter == 1;
+    run.stages = 0;
+    run.out = dev[0];
+    run.st_out = state[0];
+    run.part_out = part[0];
+    if (!hip_ok(launch_step1d(s, run, st), "1D step kernel")) return DGX_EDEVICE;
+  }
+  int hs[4] = {0, 0, 0, 0};
+  double hd[2] = {0, 0};  // Dt, T
+  int queued = 0, chunk = 16;
+  for (;;) {
+    const int k = nsteps > 0 ? std::min(chunk, nsteps - queued) : chunk;
+    if (k <= 0) break;
+    for (int i = 0; i < k; ++i, ++queued) {
+      KernelTimer kt(s, 4, st);
+      const int p = queued & 1;
+      Step1DRun run;
+      run.In = buf[p];
+      run.Out = buf[p ^ 1];
+      run.limited = limiter == 1;
+      run.part_in = part[p];
+      run.npart = nblk;
+      run.cfl = cfl;
+      run.tf = tf;
+      run.in = dev[p];
+      run.out = dev[p ^ 1];
+      run.st_in = state[p];
+      run.st_out = state[p ^ 1];
+      run.part_out = part[p ^ 1];
+      if (!hip_ok(launch_step1d(s, run, st), "1D step kernel")) return DGX_EDEVICE;
+    }
+    const int p = queued & 1;
+    if (!hip_ok(hipMemcpyAsync(hs, state[p], sizeof(hs), hipMemcpyDeviceToHost, st), "time state readback") ||
+        !hip_ok(hipMemcpyAsync(hd, dev[p], sizeof(hd), hipMemcpyDeviceToHost, st), "time readback") ||
+        !hip_ok(hipStreamSynchronize(st), "time readback"))
+      return DGX_EDEVICE;
+    if (hs[0] || hs[1]) break;
+    const double left = (tf - hd[1]) / hd[0];
+    chunk = left < 1 ? 1 : (int)std::min(256.0, std::ceil(left) + 1);
+  }
+  *n_out_steps = hs[3];
+  *T_out = hd[1];
+  const dgx_status r = copy_state(s, U, buf[hs[3] & 1], st);
+  if (r != DGX_OK) return r;
+  return hs[2] ? fail(DGX_EDT, "time step too small or NaN (rk.cc:147-148)") : DGX_OK;
+}
+
 // RK::RK_integration's CFL branch (rk.cc:100-233): the initial limit, then
 // per step Dt from CFL (one 8-byte read-back, as DtFromCFL's, rk.cc:265-268),
 // the stop on a tiny or NaN Dt (rk.cc:147-148), the clamps to the final time
@@ -687,8 +784,11 @@ static dgx_status integrate_cfl(Solver& s, double* U, double cfl, int nsteps, co
     *n_out_steps = n;
     *T_out = T;
   };
+  const bool device_timed = s.device_time && !on_output && n_out == 1 && (limiter == 0 || limiter == 1);
+  if (device_timed && s.step1d(limiter))
+    return integrate_cfl_step1d(s, U, cfl, nsteps, tf, limiter, n_out_steps, T_out, st);
   if ((r = do_limit(s, limiter, U, st)) != DGX_OK) return r;
-  if (s.device_time && !on_output && n_out == 1 && (limiter == 0 || limiter == 1))
+  if (device_timed)
     return integrate_cfl_device(s, U, cfl, nsteps, tf, limiter, n_out_steps, T_out, st);
   bool done = false;
   while (!done && (nsteps <= 0 || n < nsteps)) {
@@ -747,10 +847,18 @@ dgx_status dgx_rk4_integrate(dgx_solver* h, double* U, int mode, double dt_or_cf
     if (!hip_ok(hipMemcpyAsync(dt_dev, &dt_or_cfl, sizeof(double), hipMemcpyHostToDevice, st), "dt upload") ||
         !hip_ok(hipStreamSynchronize(st), "dt upload"))
       return DGX_EDEVICE;
+    double* cur = U;
     for (; n < nsteps; ++n) {
-      if ((r = rk4_step(s, U, dt_dev, limiter, st)) != DGX_OK) return r;
+      if (s.step1d(limiter)) {  // one launch per step, U and Ustar in turn
+        double* out = cur == U ? s.Ustar : U;
+        if ((r = step1d_fixed(s, cur, out, dt_dev, limiter, st)) != DGX_OK) return r;
+        cur = out;
+      } else if ((r = rk4_step(s, U, dt_dev, limiter, st)) != DGX_OK) {
+        return r;
+      }
       T = T + dt_or_cfl;
     }
+    if ((r = copy_state(s, U, cur, st)) != DGX_OK) return r;
   } else if (mode == 1) {
     r = integrate_cfl(s, U, dt_or_cfl, nsteps, &tf, 1, limiter, nullptr, nullptr, &n, &T, st);
     if (r != DGX_OK) {

@@ -54,10 +54,12 @@ struct DevTables {
 };
 
 // Cartesian meshes whose faces follow the structured pattern (element
-// e = ey*nx + ex, side 0 = left/lower element) run the fused tile kernel of
-// stage.hip, which finds faces from the tile structure and reads their
-// normals and Jacobians from per-face arrays in grid order.
+// e = ey*nx + ex, side 0 = left/lower element; grid) find faces from the
+// grid structure and read their normals and Jacobians from per-face arrays in
+// grid order.  on: their sides are whole tiles too, and the fused tile kernel
+// of stage.hip is the kernel path.
 struct Cart {
+  bool grid = false;
   bool on = false;
   int nx = 0, ny = 1, tx = 1, ty = 1;
   int bc[4] = {0, 0, 0, 0};
@@ -96,8 +98,12 @@ struct Solver {
   int* sens_changed = nullptr;  // [kRelaxBatch] change flags of a batch of sensor relaxation sweeps
   int* flag_list = nullptr; // [N_E] flagged elements (launch_limit_flagged)
   double* m2buf = nullptr;  // m2 limiting: 15 per-field arrays of N_E*N_s (allocated on first use)
-  double* dscratch = nullptr;  // device scalars: [1] Dt, [2] the time of a device-timed CFL run
-  int* time_state = nullptr;   // device-timed CFL run: stop, last step taken, Dt error, steps (k_dt_step)
+  double* dscratch = nullptr;  // device scalars: [1] Dt, [2] the time of a device-timed CFL run; [4..7] {Dt, T} in two slots (1D)
+  int* time_state = nullptr;   // device-timed CFL run: stop, last step taken, Dt error, steps (k_dt_step); two slots
+  double* part1d = nullptr;    // 1D whole-step kernel: two slots of part1d_len per-block maxima of |u|+a and node 0's, then two doubles
+  int part1d_len = 0;
+  // 1D grids run whole RK4 steps in one launch (step1d.hip) with limiters 0 and 1
+  bool step1d(int limiter) const { return part1d && path != PATH_GENERAL && (limiter == 0 || limiter == 1); }
   const int* gate = nullptr;   // while steps of such a run are enqueued: time_state, read by their kernels
   bool device_time = true;     // CFL runs without outputs keep their time control on the device
   double* cons_partial = nullptr;  // conservation totals: per-block double-double partial sums
@@ -142,6 +148,30 @@ bool stage_tiles(int D, int nx, int ny, int* tx, int* ty);
 hipError_t launch_stage(const Solver& s, int mode, int stage, const double* Uin, const double* Un, double* Uacc,
                         double* Uout, const double* dt_dev, double* f_out, hipStream_t st, double* means = nullptr,
                         double* uavg = nullptr, double* psens = nullptr, bool* means_done = nullptr);
+// 1D whole RK4 step (step1d.hip): the shape of its launch, and one launch.
+// Dt: *dt_fixed, or from part_in with the
+// time control in {in, st_in} -> {out, st_out}; stages 0: only the limiter
+// (and the start of a run's time control when st_out is given).
+struct Step1DShape {
+  int lanes, threads, R, blocks, own;
+};
+Step1DShape step1d_shape(int P, int NE, bool limited);
+struct Step1DRun {
+  const double* In = nullptr;
+  double* Out = nullptr;
+  bool limited = false;
+  int stages = 4;
+  const double* dt_fixed = nullptr;
+  const double* part_in = nullptr;
+  int npart = 0;
+  double cfl = 0, tf = 0;
+  const double* in = nullptr;
+  double* out = nullptr;
+  const int* st_in = nullptr;
+  int* st_out = nullptr;
+  double* part_out = nullptr;
+};
+hipError_t launch_step1d(const Solver& s, const Step1DRun& r, hipStream_t st);
 hipError_t launch_upa_max(const Solver& s, const double* U, double cfl, double* dt_dev, hipStream_t st);
 // one step's Dt on the device with the stop, final-time clamp and step count
 // of a CFL run (k_dt_step): state = Solver::time_state, T_dev its time
