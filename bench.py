@@ -21,8 +21,7 @@ fixed Dt from CFL 0.3; `sod`, the 1D single-fluid Sod tube on 1000 elements,
 p=2, Rusanov, HR limiter, CFL 0.4 steps (Dt from the state every step);
 `ensemble`, 256 independent 1D two-fluid Riemann problems (element counts
 uniform in [200, 4000], orders uniform in {1, 2, 3}, seeded states), Roe, HR
-limiter, each with its own CFL 0.4 step, advanced by one graph launch of K
-steps.  `--precision` and `--limiter` select another form (on `bubble`:
+limiter, each with its own CFL 0.4 step, advanced by one call of K steps.  `--precision` and `--limiter` select another form (on `bubble`:
 `--precision fp64 --limiter hr` is the plain form alone).
 
     python bench.py [--steps K] [--warmup W] [--config bubble|vortex|sod|ensemble] [--no-cpu-baseline]
@@ -300,7 +299,7 @@ def main() -> int:
 
 def bench_ensemble(args, device):
     """The batched ensemble: autotune, W warmup steps, then K steps timed as
-    one graph launch.  DOF-updates count the problems that completed every
+    one call.  DOF-updates count the problems that completed every
     step (status 0); strong random Riemann problems can lose positivity and
     stop, as they would in the reference."""
     import numpy as np
@@ -335,7 +334,7 @@ def bench_ensemble(args, device):
         "vs_baseline": None, "dtype": "f64", "data": "synthetic",
         "config": {"workload": "256 independent 1D two-fluid Riemann problems (N_E uniform in [200,4000], p uniform "
                                "in {1,2,3}, rho,p log-uniform [0.1,10], u in [-2,2], gamma in [1.1,1.7] per side), "
-                               "Roe, HR limiter, per-problem Dt from CFL 0.4, one graph launch of K steps",
+                               "Roe, HR limiter, per-problem Dt from CFL 0.4, one call of K steps",
                    "problems": n, "dofs": int(dofs.sum()), "completed": int(ok.sum()),
                    "block_sizes": batch.block_sizes, "parallelism": "single GPU"},
         "step_roofline": {"c": 16 + 8, "achieved": 24 * 8.0 * float(dofs[ok].sum()) / (elapsed / args.steps) / 1e9,

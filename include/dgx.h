@@ -278,14 +278,10 @@ void dgx_batch_free(dgx_batch* b);
  * Each problem's slice uses the usual layout U[(e*N_F+f)*N_s+i]. */
 long dgx_batch_state_offset(const dgx_batch* b, int k);
 /* sizes[0] = workgroup size, sizes[1] = workgroups of a launch, sizes[2] =
- * problems cut into chunks.  Without a cut problem every problem has its own
- * workgroup, largest first.  A problem whose work (N_E times a measured cost
- * per element of order p) is well above
- * the ensemble's average per resident workgroup, and that has at least two
- * chunks' elements (dgx_batch_set_min_chunk), is cut into chunks of
- * consecutive elements on consecutive workgroups; the other problems then
- * share the remaining resident workgroups, longest first to the least
- * loaded.  Cut or not, every problem gets the same bits. */
+ * problems cut into chunks.  A problem of more elements than a workgroup's
+ * window holds is cut into chunks of consecutive elements, one workgroup
+ * each, of at least dgx_batch_set_min_chunk elements.  Cut or not, every
+ * problem gets the same bits. */
 dgx_status dgx_batch_block_sizes(dgx_batch* b, int* sizes);
 /* Elements per chunk at least (default 64; 0: no problem is cut; else >= 8). */
 dgx_status dgx_batch_set_min_chunk(dgx_batch* b, int min_chunk);
@@ -295,14 +291,12 @@ dgx_status dgx_batch_set_block_sizes(dgx_batch* b, const int* sizes);
  * fastest of two timed runs after a warm-up run) on scratch copies of U (U is
  * not modified) and keeps the fastest size. */
 dgx_status dgx_batch_autotune(dgx_batch* b, const double* U, double cfl, int limiter, void* stream);
-/* nsteps RK4 steps of every problem in one graph launch.  Problem k uses
+/* nsteps RK4 steps of every problem, one launch per step.  Problem k uses
  * Dt = cfl*Dx_k/(2p_k+1)/max(|u|+a) (deck CFL scaling, main.cc:896-897);
  * limiter 0 none or 1 hrl; limit_initial limits the initial state first
  * (rk.cc:100-114).  T (double[n], device) accumulates each problem's time;
  * status (int[n], device, zero on entry) becomes 1 for a problem whose Dt
- * fell below 1e-14 or was NaN (rk.cc:147-148); that problem stops.  Status 2
- * marks a cut problem whose chunks stopped waiting for each other (a bounded
- * wait that timed out; not expected when the device runs nothing else). */
+ * fell below 1e-14 or was NaN (rk.cc:147-148); that problem stops. */
 dgx_status dgx_batched_rk4(dgx_batch* b, double* U, double cfl, int nsteps, int limiter, int limit_initial,
                            double* T, int* status, void* stream);
 
