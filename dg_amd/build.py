@@ -35,6 +35,8 @@ SOURCES = [
     ("capi.cc", "hip-host", []),
     ("rhs.hip", "hipcc", []),
     ("stage.hip", "hipcc", []),
+    ("stage_multifluid.hip", "hipcc", []),
+    ("stage_passive_stiffened.hip", "hipcc", []),
     ("step1d.hip", "hipcc", []),
     ("batch.hip", "hipcc", []),
     ("mlp.hip", "hipcc", []),

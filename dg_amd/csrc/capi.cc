@@ -112,20 +112,34 @@ dgx_status fail(int code, const std::string& msg) {
 // pattern the grid kernels assume (element e = ey*nx + ex; side 0 is the
 // left/lower element, or the boundary element of a boundary face; closures
 // and periodic partners as built by build_tables; normals along the axes)
-// and gathers each face's normal and Jacobians into grid order.  Any
-// mismatch leaves the general path.  True when its sides are whole tiles
+// (k_face_geometry gathers their geometry into grid order).  Any mismatch
+// leaves the general path.  True when its sides are whole tiles
 // too; out.grid when only the pattern holds.
 bool cartesian_layout(const Tables& t, Cart& out) {
   Cart c;
-  const int D = t.D, nx = t.nx, ny = (D == 2) ? t.ny : 1;
-  if (nx * ny != t.N_E) return false;
-  const bool whole_tiles = stage_tiles(D, nx, ny, &c.tx, &c.ty);
+  const int D = t.D, NN = t.N_N;
+  // a mesh read from a file: the length of its first row, if its elements are
+  // in grid order, and the boundary tags of its first and last elements
+  const bool from_file = t.nx == 0;
+  int nx = t.nx;
+  if (from_file)
+    for (nx = 1; nx < t.N_E && t.neighbors[(size_t)(nx - 1) * NN + 1] == nx; ++nx) {}
+  const int ny = D == 2 ? (from_file ? t.N_E / nx : t.ny) : 1;
+  if ((long)nx * ny != t.N_E) return false;
+  const bool whole_tiles = stage_tiles(D, nx, ny, &c.tx, &c.ty) && !from_file;
   c.nx = nx;
   c.ny = ny;
   for (int k = 0; k < 4; ++k) c.bc[k] = t.bc[k];
-  c.gx.assign((size_t)(nx + 1) * ny * 4, 0.0);
-  c.gy.assign(D == 2 ? (size_t)nx * (ny + 1) * 4 : 4, 0.0);
-  std::vector<char> seen_x((size_t)(nx + 1) * ny, 0), seen_y(D == 2 ? (size_t)nx * (ny + 1) : 0, 0);
+  if (from_file)
+    for (int f = 0; f < t.M_T; ++f) {
+      if (t.face_tag[f] == 0) continue;
+      const int e = t.face_elem[2 * f], cl = t.face_closure[2 * f];
+      const int side = D == 1 ? cl : (cl == 3 ? 0 : cl == 1 ? 1 : cl == 0 ? 2 : 3);
+      if (e == 0 || e == t.N_E - 1) c.bc[side] = t.face_tag[f];  // every other face is checked against these below
+    }
+  const size_t nfx = (size_t)(nx + 1) * ny;
+  std::vector<char> seen(nfx + (D == 2 ? (size_t)nx * (ny + 1) : 0), 0);
+  size_t found = 0;
   const bool perx = c.bc[0] == BC_PERIODIC, pery = D == 2 && c.bc[2] == BC_PERIODIC;
   for (int f = 0; f < t.M_T; ++f) {
     const int e0 = t.face_elem[2 * f], c0 = t.face_closure[2 * f];
@@ -156,19 +170,12 @@ bool cartesian_layout(const Tables& t, Cart& out) {
     // normals of a Cartesian grid: the axis direction up to rounding
     for (int a = 0; a < D; ++a)
       if (!(std::fabs(t.normals[(size_t)f * D + a] - wn[a]) <= 1e-6)) return false;
-    std::vector<char>& seen = xface ? seen_x : seen_y;
-    if (seen[slot]) return false;
-    seen[slot] = 1;
-    double* g = (xface ? c.gx.data() : c.gy.data()) + slot * 4;
-    g[0] = t.normals[(size_t)f * D];
-    g[1] = (D == 2) ? t.normals[(size_t)f * D + 1] : 0.0;
-    g[2] = t.JF[2 * f];
-    g[3] = t.JF[2 * f + 1];
+    char& mark = seen[xface ? slot : nfx + slot];
+    if (mark) return false;
+    mark = 1;
+    ++found;
   }
-  for (char v : seen_x)
-    if (!v) return false;
-  for (char v : seen_y)
-    if (!v) return false;
+  if (found != seen.size()) return false;
   c.grid = true;
   c.on = whole_tiles;
   out = std::move(c);
@@ -302,7 +309,16 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
   {
     double mmax = 0.0;
     for (int k = 0; k < Ns * Ns; ++k) mmax = std::max(mmax, std::fabs(t.Minv[k]));
+    // the mesh builder inverts one matrix per distinct Jacobian, so elements
+    // with the same bits of J have the same matrix: each value is checked once
+    // (or again, where another took its place in the table)
+    std::vector<double> seen(4096, 0.0);
     for (int e = 1; e < NE && uniform_minv; ++e) {
+      uint64_t bits;
+      std::memcpy(&bits, &t.J[e], 8);
+      double& slot = seen[(bits ^ (bits >> 12) ^ (bits >> 24)) & 4095];
+      if (slot == t.J[e]) continue;
+      slot = t.J[e];
       const double r = t.J[0] / t.J[e];
       const double* Me = &t.Minv[(size_t)e * Ns * Ns];
       for (int k = 0; k < Ns * Ns; ++k)
@@ -354,8 +370,9 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
             upload(s, &s.t.neighbors, t.neighbors.data(), t.neighbors.size()) &&
             upload(s, &s.t.weight, t.weight.data(), t.weight.size());
   if (ok && s.cart.grid)
-    ok = upload(s, &s.t.face_geo_x, s.cart.gx.data(), s.cart.gx.size()) &&
-         upload(s, &s.t.face_geo_y, s.cart.gy.data(), s.cart.gy.size());
+    ok = alloc(s, &s.t.face_geo_x, (size_t)(s.cart.nx + 1) * s.cart.ny * 4) &&
+         alloc(s, &s.t.face_geo_y, D == 2 ? (size_t)s.cart.nx * (s.cart.ny + 1) * 4 : 4) &&
+         hip_ok(launch_face_geometry(s, nullptr), "face geometry") && hip_ok(hipStreamSynchronize(nullptr), "face geometry");
   if (ok && D == 1)
     ok = upload(s, &s.t.Lag2Mono, t.Lag2Mono.data(), t.Lag2Mono.size()) &&
          upload(s, &s.t.Mono2Lag, t.Mono2Lag.data(), t.Mono2Lag.size());
@@ -366,9 +383,8 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
          upload(s, &s.t.Lag2MonoY, t.Lag2MonoY.data(), t.Lag2MonoY.size()) &&
          upload(s, &s.t.MonoX2Lag, t.MonoX2Lag.data(), t.MonoX2Lag.size());
   s.hr_const = D == 2 && s.P <= 2 && hr_tables_match(s.P, t.Lag2MonoX.data(), t.MonoX2MonoY.data(), t.MonoY2Lag.data());
-  // k_hr2d's tiles are 8 x 8 or 8 x 4 elements whatever the stage tile
-  if (s.cart.on && s.hr_const && s.NF <= 5 && s.cart.nx % 8 == 0 && s.cart.ny % 4 == 0) {
-    // the one-launch HR limiter assumes e -/+ 1 and e -/+ nx inside a tile,
+  if (s.cart.grid && s.hr_const && s.NF <= 5) {
+    // the one-launch HR limiter assumes e -/+ 1 and e -/+ nx inside the grid,
     // takes the rows below and above it and the ends of every row from the
     // table, and takes the x neighbours of a halo-row element to be the halo
     // elements of the x neighbours (p = 3 would not fit its LDS: two sweeps);
@@ -399,7 +415,7 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
        alloc(s, &s.dscratch, 8) && alloc(s, &s.time_state, 8) &&
        alloc(s, &s.cons_partial, conservation_scratch_doubles()) &&
        alloc(s, &s.dt_partial, ((size_t)NE * Ns + 255) / 256 + 1) &&
-       ((!s.cart.on && D != 1) || alloc(s, &s.Ustar2, S));
+       ((!s.cart.grid && D != 1) || alloc(s, &s.Ustar2, S));
   // the 1D whole-step kernel: one shared mass matrix (to J), both ends
   // periodic or neither
   if (ok && D == 1 && s.cart.grid && uniform_minv &&
@@ -429,7 +445,7 @@ dgx_status dgx_rhs(dgx_solver* h, const double* U, double* f_rk, void* stream) {
   if (!h || !U || !f_rk) return fail(DGX_EINVAL, "dgx_rhs: null argument");
   Solver& s = h->s;
   hipStream_t st = as_stream(stream);
-  if (s.tiled())
+  if (s.stage_kernel())
     return hip_ok(launch_stage(s, 0, 0, U, U, nullptr, nullptr, nullptr, f_rk, st), "dgx_rhs tile kernel")
                ? DGX_OK
                : DGX_EDEVICE;
@@ -576,7 +592,7 @@ static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, 
     if ((r = step1d_fixed(s, U, s.Ustar, dt, limiter, st)) != DGX_OK) return r;
     return copy_state(s, U, s.Ustar, st);
   }
-  if (DGX_RK_HR2D && limiter == 1 && ((s.tiled() && s.hr2d) || s.D == 1)) {
+  if (DGX_RK_HR2D && limiter == 1 && ((s.stage_kernel() && s.hr2d) || s.D == 1)) {
     // One-launch HR limiter (out of place; 2D tiles, or 1D): every stage
     // writes Ustar, the limiter takes Ustar to Ustar2 (the next stage's input)
     // and, after the last stage, to U.  U keeps the step's initial state
@@ -587,7 +603,7 @@ static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, 
         if ((r = timed_hr_oop(s, s.Ustar, s.Ustar2, st)) != DGX_OK) return r;
         Uin = s.Ustar2;
       }
-      if (s.tiled()) {
+      if (s.stage_kernel()) {
         KernelTimer kt(s, 4, st);
         if (!hip_ok(launch_stage(s, 1, k, Uin, U, s.Uacc, s.Ustar, dt, nullptr, st), "tile kernel"))
           return DGX_EDEVICE;
@@ -607,7 +623,7 @@ static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, 
   // blocks write their stage output, so its stages ping-pong between two
   // buffers (U -> Ustar -> Ustar2 -> Ustar -> U); the face + element path
   // consumes all traces in the face kernel and updates Ustar in place.
-  const bool tiled = s.tiled();
+  const bool tiled = s.stage_kernel();
   // with the learned indicator the tile kernel also writes its output's cell
   // means, and the indicator that follows skips its own pass over the state
   double* means = (limiter == 8 && s.mlp && s.fuse_means) ? s.mlp_avg : nullptr;

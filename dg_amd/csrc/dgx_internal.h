@@ -56,14 +56,15 @@ struct DevTables {
 // Cartesian meshes whose faces follow the structured pattern (element
 // e = ey*nx + ex, side 0 = left/lower element; grid) find faces from the
 // grid structure and read their normals and Jacobians from per-face arrays in
-// grid order.  on: their sides are whole tiles too, and the fused tile kernel
-// of stage.hip is the kernel path.
+// grid order.  on: built as such, with sides of whole tiles, and the tile
+// kernel of stage.cuh is the kernel path; meshes read from a file in grid
+// order, and sides of other lengths, use it too unless the face + element
+// kernels are asked for.
 struct Cart {
   bool grid = false;
   bool on = false;
   int nx = 0, ny = 1, tx = 1, ty = 1;
   int bc[4] = {0, 0, 0, 0};
-  std::vector<double> gx, gy;  // host copies of DevTables::face_geo_x / face_geo_y
 };
 
 enum KernelPath { PATH_AUTO = 0, PATH_GENERAL = 1, PATH_TILED = 2 };
@@ -81,7 +82,16 @@ struct Solver {
   int path = PATH_AUTO;
   int precision = 0;  // tile kernel: 0 FP64, 1 FP32-MFMA map/integrate (2D p=2)
   bool tiled() const { return cart.on && path != PATH_GENERAL; }
-  bool hr2d = false;  // 2D tile layout whose neighbour table follows it: one-launch HR limiter (k_hr2d)
+  // runs the tile kernel: the kernel path `tiled`, or a 2D grid whose sides are
+  // not whole tiles unless the face + element kernels are asked for.  Measured,
+  // tile against face + element kernels: 500x500 p=2 single fluid 0.50 against
+  // 0.74 ms a step, 450x225 p=1 two-fluid 0.25 against 0.31 (with the one-launch
+  // limiter); p = 3 with five fields and more fills a CU's LDS with one tile
+  // and measured 0.82x.
+  bool stage_kernel() const {
+    return tiled() || (cart.grid && D == 2 && path != PATH_GENERAL && !(P == 3 && NF > 4));
+  }
+  bool hr2d = false;  // 2D grid whose neighbour table follows it: one-launch HR limiter (k_hr2d)
   bool hr_const = false;  // 2D p <= 2 with the HR transforms of hr_tables.h: constant-table sweeps
   // work buffers
   double* Qe = nullptr;     // face contributions, element-major [((e*N_N+k)*NF+f)*M_s+j]
@@ -139,6 +149,8 @@ hipError_t launch_face(const Solver& s, const double* U, hipStream_t st);
 // mode 0: f_rk = S+F+Q to out; mode 1: RK stage `stage` update (see rhs.hip)
 hipError_t launch_elem(const Solver& s, int mode, int stage, const double* Uin, const double* Un, double* Uacc,
                        double* Uout, const double* dt_dev, double* f_out, hipStream_t st);
+// DevTables::face_geo_x / face_geo_y of a grid from its normals and JF
+hipError_t launch_face_geometry(const Solver& s, hipStream_t st);
 // fused tile kernel (Cartesian meshes): same modes as launch_elem
 bool stage_tiles(int D, int nx, int ny, int* tx, int* ty);
 // means: also write the output tile's cell means of rho, p and alpha there

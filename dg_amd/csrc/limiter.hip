@@ -271,9 +271,11 @@ __global__ __launch_bounds__(256) void k_hr_sweep_c(int N_E, int NF, int N_N, co
 // intermediate state never reaches HBM.  In and Out must differ:
 // neighbouring tiles read In's rows.  At least six waves per SIMD (three
 // 512-thread blocks of the 2D p=2 five-field limiter per CU).
-template <int Ns, int N, int SL, int NF, int TXE, int TYE, int BS, bool OUT_VEC2>
+// RAG: the grid's sides need not be whole tiles; a tile at its right or upper
+// end then holds cols x rows elements, and what lies beyond is absent.
+template <int Ns, int N, int SL, int NF, int TXE, int TYE, int BS, bool OUT_VEC2, bool RAG>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_hr2d(
-    int nx, int N_N, const int* __restrict__ nb, const double* __restrict__ In, double* __restrict__ Out,
+    int nx, int ny, int N_N, const int* __restrict__ nb, const double* __restrict__ In, double* __restrict__ Out,
     const int* gate) {
   if (gate && *gate) return;
   constexpr int ROWS = TYE + 2, W = TXE + 2, EL = NF * Ns, ROW_OUT = TXE * EL;
@@ -284,8 +286,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_
   // nodal values, then Taylor-x [row][col][f]; then Taylor-y [row][i][f]; then the output [j][i][f]
   __shared__ __align__(16) double sA[ROWS * W * EL];
   __shared__ int sE[ROWS * W];  // element of each slot, -1 if absent
-  const int tiles_x = nx / TXE;
+  const int tiles_x = RAG ? (nx + TXE - 1) / TXE : nx / TXE;
   const int ex0 = (blockIdx.x % tiles_x) * TXE, ey0 = (blockIdx.x / tiles_x) * TYE;
+  const int cols = RAG ? min(TXE, nx - ex0) : TXE, rows = RAG ? min(TYE, ny - ey0) : TYE;
   // slot elements: row 0 below the tile, rows 1..TYE the tile, row TYE+1
   // above; columns 0 and W-1 the left and right neighbours of the row's end
   // elements.  One thread per slot, so that no thread waits for more than the
@@ -293,12 +296,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_
   static_assert(ROWS * W <= BS, "one thread per slot");
   if (threadIdx.x < ROWS * W) {
     const int c = threadIdx.x % W, r = threadIdx.x / W;
-    const int i = c == 0 ? 0 : (c == W - 1 ? TXE - 1 : c - 1);  // the row element it starts from
-    int e;
-    if (r == 0) e = nb[(ey0 * nx + ex0 + i) * N_N + 2];
-    else if (r == ROWS - 1) e = nb[((ey0 + TYE - 1) * nx + ex0 + i) * N_N + 3];
-    else e = (ey0 + r - 1) * nx + ex0 + i;
-    if (c == 0 || c == W - 1) e = e >= 0 ? nb[e * N_N + (c == 0 ? 0 : 1)] : -1;
+    const int i = c == 0 ? 0 : (c == cols + 1 ? cols - 1 : c - 1);  // the row element it starts from
+    int e = -1;
+    if (!RAG || (c <= cols + 1 && r <= rows + 1)) {
+      if (r == 0) e = nb[(ey0 * nx + ex0 + i) * N_N + 2];
+      else if (r == rows + 1) e = nb[((ey0 + rows - 1) * nx + ex0 + i) * N_N + 3];
+      else e = (ey0 + r - 1) * nx + ex0 + i;
+      if (c == 0 || c == cols + 1) e = e >= 0 ? nb[e * N_N + (c == 0 ? 0 : 1)] : -1;
+    }
     sE[threadIdx.x] = e;
   }
   __syncthreads();
@@ -308,8 +313,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_
   constexpr int TOT = ROWS * W * EL, PER = (TOT + BS - 1) / BS;
   const int t2 = threadIdx.x;
   const int f2 = t2 % NF, i2 = (t2 / NF) % TXE, r2 = t2 / (NF * TXE);
-  const bool on2 = t2 < ROWS * TXE * NF && sE[r2 * W + i2 + 1] >= 0;
-  const bool on3 = t2 < TYE * TXE * NF;
+  const bool on2 = t2 < ROWS * TXE * NF && (!RAG || i2 < cols) && sE[r2 * W + i2 + 1] >= 0;
+  const bool on3 = t2 < TYE * TXE * NF && (!RAG || (i2 < cols && r2 < rows));
   double v[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
@@ -402,18 +407,21 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_
   }
   __syncthreads();
   // pairs of doubles when Out is 16-byte aligned (every row start then is:
-  // nx and ex0 are multiples of TXE), else single doubles.  A template
+  // nx and ex0 are multiples of TXE or, RAG, the host has found nx*NF*Ns and
+  // NF*Ns*cols even), else single doubles.  A template
   // parameter, not a run-time branch: the branch cost two VGPRs, one wave
   // per SIMD and 25 % of the time.
   if constexpr (OUT_VEC2) {
     const double2* so = reinterpret_cast<const double2*>(sA);
     for (int q = threadIdx.x; q < TYE * ROW_OUT / 2; q += BS) {
       const int j = q / (ROW_OUT / 2), r = q - j * (ROW_OUT / 2);
+      if (RAG && (j >= rows || 2 * r >= cols * EL)) continue;
       reinterpret_cast<double2*>(Out + ((long)(ey0 + j) * nx + ex0) * EL)[r] = so[q];
     }
   } else {
     for (int q = threadIdx.x; q < TYE * ROW_OUT; q += BS) {
       const int j = q / ROW_OUT, r = q - j * ROW_OUT;
+      if (RAG && (j >= rows || r >= cols * EL)) continue;
       Out[((long)(ey0 + j) * nx + ex0) * EL + r] = sA[q];
     }
   }
@@ -1160,7 +1168,7 @@ hipError_t launch_limit_hr(Solver& s, double* U, hipStream_t st) {
 }
 
 // Out = HR(In) with both 2D sweeps in one launch (k_hr2d), p <= 2; needs the
-// tile layout and a neighbour table that follows it (Solver::hr2d).
+// grid layout and a neighbour table that follows it (Solver::hr2d).
 hipError_t launch_limit_hr_oop(Solver& s, const double* In, double* Out, hipStream_t st) {
   if (In == Out) return hipErrorInvalidValue;
   if (s.D == 1) {
@@ -1184,23 +1192,30 @@ hipError_t launch_limit_hr_oop(Solver& s, const double* In, double* Out, hipStre
   // per output column) and ran 167 against 177 us on the 1024 x 512 p = 2
   // two-fluid state
   constexpr int TXE = 8;
-  // every element must lie in a tile (the eligibility check, Solver::hr2d, asks the same)
-  if (s.cart.nx % TXE != 0 || s.cart.ny % 4 != 0) return hipErrorInvalidValue;
-  const int tye = s.cart.ny % 8 == 0 ? 8 : 4;
-  const int tiles = (s.cart.nx / TXE) * (s.cart.ny / tye);
+  // grids whose sides are not whole tiles: 8 x 8 ones that reach past the ends
+  const bool ragged = s.cart.nx % TXE != 0 || s.cart.ny % 4 != 0;
+  const int tye = ragged || s.cart.ny % 8 == 0 ? 8 : 4;
+  const int tiles = ((s.cart.nx + TXE - 1) / TXE) * ((s.cart.ny + tye - 1) / tye);
   return by_order_ns(s.D, s.P, [&](auto d, auto p) -> hipError_t {
     constexpr int D = decltype(d)::value, P = decltype(p)::value;
     if constexpr (D == 2 && P <= 2) {
       constexpr int Ns = Shape<D, P>::Ns, SL = P + 1;
       auto go = [&](auto nf, auto ty) -> hipError_t {
         constexpr int NF = decltype(nf)::value, TYE = decltype(ty)::value, BS = TYE == 4 ? 256 : 512;
-        if ((reinterpret_cast<uintptr_t>(Out) & 15) == 0)
-          hipLaunchKernelGGL((k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, true>), dim3(tiles), dim3(BS), 0, st, s.cart.nx,
-                             s.N_N, s.t.neighbors, In, Out, s.gate);
-        else
-          hipLaunchKernelGGL((k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, false>), dim3(tiles), dim3(BS), 0, st, s.cart.nx,
-                             s.N_N, s.t.neighbors, In, Out, s.gate);
-        return hipGetLastError();
+        const bool vec = (reinterpret_cast<uintptr_t>(Out) & 15) == 0;
+        auto run = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(tiles), dim3(BS), 0, st, s.cart.nx, s.cart.ny, s.N_N, s.t.neighbors, In, Out,
+                             s.gate);
+          return hipGetLastError();
+        };
+        if constexpr (TYE == 8) {
+          if (ragged)
+            return vec && (NF * Ns % 2 == 0 || s.cart.nx % 2 == 0)
+                       ? run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, true, true>)
+                       : run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, false, true>);
+        }
+        return vec ? run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, true, false>)
+                   : run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, false, false>);
       };
       using I4 = std::integral_constant<int, 4>;
       using I5 = std::integral_constant<int, 5>;
