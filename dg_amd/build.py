@@ -29,14 +29,18 @@ HIP_FLAGS = [
     "-Wno-unused-result",
 ]
 
+# matrix results in ordinary registers: without it the stage kernels copy each
+# through an accumulation register (88 moves and 24 registers at 2D p=2 two-fluid)
+MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+
 SOURCES = [
     # (source, compiler, extra flags)
     ("mesh.cc", "cxx", []),
     ("capi.cc", "hip-host", []),
-    ("rhs.hip", "hipcc", []),
-    ("stage.hip", "hipcc", []),
-    ("stage_multifluid.hip", "hipcc", []),
-    ("stage_passive_stiffened.hip", "hipcc", []),
+    ("rhs.hip", "hipcc", MFMA_VGPR),
+    ("stage.hip", "hipcc", MFMA_VGPR),
+    ("stage_multifluid.hip", "hipcc", MFMA_VGPR),
+    ("stage_passive_stiffened.hip", "hipcc", MFMA_VGPR),
     ("step1d.hip", "hipcc", []),
     ("batch.hip", "hipcc", []),
     ("mlp.hip", "hipcc", []),

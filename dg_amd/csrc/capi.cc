@@ -108,6 +108,40 @@ dgx_status fail(int code, const std::string& msg) {
 }
 
 
+// The 1D tables of the 2D p = 2 element for vol_tensor_wave, [table][k*4 + j]:
+// the Lagrange polynomials at the Gauss points V[point j][node k], their
+// derivatives, both times the point's weight as [point k][node j], and the
+// inverse mass matrix of [-1, 1].  The points and weights are those of the 2D
+// tables (weight = product of the 1D ones, which add up to 2).
+std::vector<double> tensor_tables(const Tables& t) {
+  std::vector<double> out(5 * 16, 0.0);
+  std::vector<double> x;
+  for (int g = 0; g < t.N_G; ++g) {
+    bool seen = false;
+    for (double v : x) seen = seen || std::fabs(v - t.points[2 * g]) < 1e-12;
+    if (!seen) x.push_back(t.points[2 * g]);
+  }
+  std::sort(x.begin(), x.end());
+  for (int p = 0; p < 4; ++p) {
+    double w = 0.0;
+    for (int g = 0; g < t.N_G; ++g)
+      if (std::fabs(t.points[2 * g] - x[p]) < 1e-12) w += t.weight[g];
+    w *= 0.5;
+    const double z = x[p], v[3] = {0.5 * z * (z - 1.0), 1.0 - z * z, 0.5 * z * (z + 1.0)}, d[3] = {z - 0.5, -2.0 * z, z + 0.5};
+    for (int n = 0; n < 3; ++n) {
+      out[n * 4 + p] = v[n];
+      out[16 + n * 4 + p] = d[n];
+      out[32 + p * 4 + n] = v[n] * w;
+      out[48 + p * 4 + n] = d[n] * w;
+    }
+  }
+  // inverse of (1/15) [4 2 -1; 2 16 2; -1 2 4]
+  const double m[3][3] = {{4.5, -0.75, 1.5}, {-0.75, 1.125, -0.75}, {1.5, -0.75, 4.5}};
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) out[64 + i * 4 + j] = m[i][j];
+  return out;
+}
+
 // Checks that the mesh is a Cartesian grid whose faces follow the structured
 // pattern the grid kernels assume (element e = ey*nx + ex; side 0 is the
 // left/lower element, or the boundary element of a boundary face; closures
@@ -373,6 +407,10 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
     ok = alloc(s, &s.t.face_geo_x, (size_t)(s.cart.nx + 1) * s.cart.ny * 4) &&
          alloc(s, &s.t.face_geo_y, D == 2 ? (size_t)s.cart.nx * (s.cart.ny + 1) * 4 : 4) &&
          hip_ok(launch_face_geometry(s, nullptr), "face geometry") && hip_ok(hipStreamSynchronize(nullptr), "face geometry");
+  if (ok && D == 2 && t.order == 2) {
+    const std::vector<double> tt = tensor_tables(t);
+    ok = upload(s, &s.t.tensor, tt.data(), tt.size());
+  }
   if (ok && D == 1)
     ok = upload(s, &s.t.Lag2Mono, t.Lag2Mono.data(), t.Lag2Mono.size()) &&
          upload(s, &s.t.Mono2Lag, t.Mono2Lag.data(), t.Mono2Lag.size());

@@ -23,6 +23,7 @@ struct DevTables {
   // reference-element tables (column-major, as the reference)
   double *phi = nullptr, *dphi = nullptr, *phi_w = nullptr, *dphi_w = nullptr;
   double *psi = nullptr, *psi_w = nullptr;
+  double* tensor = nullptr;  // 2D p=2: 1D tables of vol_tensor_wave (tensor_tables)
   // faces
   int* face_elem = nullptr;     // [t*2+d]
   int* face_closure = nullptr;  // [t*2+d]
@@ -86,10 +87,9 @@ struct Solver {
   // not whole tiles unless the face + element kernels are asked for.  Measured,
   // tile against face + element kernels: 500x500 p=2 single fluid 0.50 against
   // 0.74 ms a step, 450x225 p=1 two-fluid 0.25 against 0.31 (with the one-launch
-  // limiter); p = 3 with five fields and more fills a CU's LDS with one tile
-  // and measured 0.82x.
+  // limiter).
   bool stage_kernel() const {
-    return tiled() || (cart.grid && D == 2 && path != PATH_GENERAL && !(P == 3 && NF > 4));
+    return tiled() || (cart.grid && D == 2 && path != PATH_GENERAL);
   }
   bool hr2d = false;  // 2D grid whose neighbour table follows it: one-launch HR limiter (k_hr2d)
   bool hr_const = false;  // 2D p <= 2 with the HR transforms of hr_tables.h: constant-table sweeps

@@ -147,6 +147,7 @@ struct ElemArgs {
   const double* __restrict__ dt;
   double* fout;
   const int* gate;  // as FaceArgs::gate
+  const double* __restrict__ tensor;  // 2D p=2: 1D tables of vol_tensor_wave
 };
 
 // One block of 256 threads handles EPB elements.  Phase 1: lane = (element,
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(256) void k_elem(ElemArgs a) {
 }
 
 // The same for 2D p=2 single-fluid and two-fluid states with the element
-// phases on the FP64 matrix cores (vol_mfma_wave): a block of 256 threads
+// phases on the FP64 matrix cores (vol_tensor_wave): a block of 256 threads
 // handles 32 consecutive elements; with the shared mass-matrix inverse the
 // wave also forms Dt*Minv*R.  Padded per-element LDS strides (a multiple of
 // 4 doubles apart for neighbouring elements: distinct bank groups).
@@ -243,30 +244,22 @@ constexpr int elem_stride(int n) { return elem_bank_ok(n) ? n : elem_stride(n + 
 template <int PH, int FL, int MODE>
 __global__ __launch_bounds__(256) void k_elem_mfma(ElemArgs a) {
   if (a.gate && *a.gate) return;
-  constexpr int D = 2, P = 2, NT = 32, NGEO = 1 + D * D;
+  constexpr int D = 2, P = 2, NT = 32;
   using V = Vol<D, P, PH>;
   constexpr int NF = V::NF, Ns = V::Ns, NU = V::NU, NQE = V::NQE;
   constexpr int SU = elem_stride(NU), SQ = elem_stride(NQE);
   __shared__ double sU[NT * SU];
   __shared__ double sQ[NT * SQ];
-  __shared__ double sW[4 * vol_wave_lds<double, PH>()];
-  __shared__ double sPhi[V::NTAB_PHI];
-  __shared__ double sDphi[PH ? V::NTAB_D : 1];
-  __shared__ double sPw[PH ? V::NTAB_PHI : 1];
-  __shared__ double sMinv[Ns * Ns];
-  __shared__ double sGeo[NT * NGEO];
+  __shared__ double sTab[kTensorTables * 16];
+  __shared__ double sGeo[NT * 4];  // J_e invJac
   __shared__ double sDte[NT];
   __shared__ int sNodeQ[18];
-  const VolTables<D, P, PH> tb{sPhi, sDphi, nullptr, sPw, sMinv};
-
   const int tid = threadIdx.x;
   const int e0 = blockIdx.x * NT;
   const int n_el = min(NT, a.N_E - e0);
   const bool uniform_minv = a.minv_stride == 0;
-  VolTableFetch<D, P, PH, false> tf;
-  tf.fetch(a.phi, a.dphi, a.phi_w, a.dphi_w, a.Minv, MODE == 1 && uniform_minv, tid);
-  constexpr int RU = (NT * NU + 255) / 256, RQ = (NT * NQE + 255) / 256, RG = (NT * NGEO + 255) / 256;
-  double ru[RU], rq[RQ], rg[RG];
+  constexpr int RU = (NT * NU + 255) / 256, RQ = (NT * NQE + 255) / 256;
+  double ru[RU], rq[RQ], rg[4], rj = 1.0;
   // elements past the end of the mesh (last block) repeat the block's first element
 #pragma unroll
   for (int r = 0; r < RU; ++r) {
@@ -278,15 +271,12 @@ __global__ __launch_bounds__(256) void k_elem_mfma(ElemArgs a) {
     const int k = tid + 256 * r, el = k / NQE;
     if (k < NT * NQE) rq[r] = a.Qe[(size_t)(e0 + (el < n_el ? el : 0)) * NQE + k % NQE];
   }
+  if (tid < NT) {
+    const int eg = (e0 + (tid < n_el ? tid : 0)) * a.geo_stride;
+    rj = a.J[eg];
 #pragma unroll
-  for (int r = 0; r < RG; ++r) {
-    const int k = tid + 256 * r, el = k / NGEO, q = k % NGEO;
-    if (k < NT * NGEO) {
-      const int eg = (e0 + (el < n_el ? el : 0)) * a.geo_stride;
-      rg[r] = q == 0 ? a.J[eg] : a.invJac[eg * D * D + q - 1];
-    }
+    for (int k = 0; k < 4; ++k) rg[k] = a.invJac[(size_t)eg * 4 + k];
   }
-  tf.store(tb, MODE == 1 && uniform_minv, tid);
   node_q_table<NF>(sNodeQ, tid);
 #pragma unroll
   for (int r = 0; r < RU; ++r) {
@@ -298,14 +288,14 @@ __global__ __launch_bounds__(256) void k_elem_mfma(ElemArgs a) {
     const int k = tid + 256 * r;
     if (k < NT * NQE) sQ[(k / NQE) * SQ + k % NQE] = rq[r];
   }
-#pragma unroll
-  for (int r = 0; r < RG; ++r) {
-    const int k = tid + 256 * r;
-    if (k < NT * NGEO) sGeo[k] = rg[r];
-  }
-  __syncthreads();
   const double dt = MODE == 1 ? a.dt[0] : 0.0;
-  if (MODE == 1 && tid < NT) sDte[tid] = uniform_minv ? dt * (a.J0 / sGeo[tid * NGEO]) : dt;
+  if (tid < NT) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sGeo[4 * tid + k] = rg[k] * rj;
+    if (MODE == 1) sDte[tid] = uniform_minv ? dt / rj : dt;
+  }
+  if (tid < kTensorTables * 16) sTab[tid] = a.tensor[tid];
+  __syncthreads();
   // RK operands of this thread's output entries, in flight during the element phases
   double pre_un[RU], pre_acc[RU];
 #pragma unroll
@@ -317,10 +307,18 @@ __global__ __launch_bounds__(256) void k_elem_mfma(ElemArgs a) {
       if (a.stage > 0) pre_acc[r] = a.Uacc[(size_t)e0 * NU + k];
     }
   }
-  __syncthreads();
   const bool wave_minv = MODE == 1 && uniform_minv;
-  vol_mfma_wave<double, PH, NT, SU, SQ, NGEO>(tb, a.dphi_w, sU, sGeo, sQ, sW, sNodeQ, tid,
-                                              wave_minv ? tb.minv : nullptr, sDte);
+  const int node = tensor_node(tid & 63);
+  const int q0 = node >= 0 ? sNodeQ[2 * node] : -1, q1 = node >= 0 ? sNodeQ[2 * node + 1] : -1;
+  auto face = [&](int el, double* qs) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      qs[f] = 0.0;
+      if (q0 >= 0) qs[f] += sQ[el * SQ + q0 + f * V::Ms];
+      if (q1 >= 0) qs[f] += sQ[el * SQ + q1 + f * V::Ms];
+    }
+  };
+  vol_tensor_wave<PH, SU>(sTab, sU, sGeo, tid, wave_minv, sDte, face);
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < RU; ++r) {
@@ -479,7 +477,7 @@ hipError_t launch_face(const Solver& s, const double* U, hipStream_t st) {
 hipError_t launch_elem(const Solver& s, int mode, int stage, const double* Uin, const double* Un, double* Uacc,
                        double* Uout, const double* dt_dev, double* f_out, hipStream_t st) {
   ElemArgs a{s.t.phi, s.t.dphi, s.t.phi_w, s.t.dphi_w, s.t.J, s.t.invJac, s.t.Minv, s.t.geo_stride,
-             s.t.minv_stride, s.t.J0, s.Qe, s.N_E, stage, Uin, Un, Uacc, Uout, dt_dev, f_out, s.gate};
+             s.t.minv_stride, s.t.J0, s.Qe, s.N_E, stage, Uin, Un, Uacc, Uout, dt_dev, f_out, s.gate, s.t.tensor};
   return dispatch(s.cfg, [&](auto d, auto p, auto ph, auto fl) -> hipError_t {
     constexpr int D = decltype(d)::value, P = decltype(p)::value, PH = decltype(ph)::value, FL = decltype(fl)::value;
     if constexpr (D == 2 && P == 2 && PH <= 1) {

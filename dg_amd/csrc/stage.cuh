@@ -41,7 +41,7 @@ struct StageArgs {
   int geo_stride, minv_stride;
   int nx, ny;
   int bc[4];  // left, right, bottom, top
-  int tiles_x, tiles_y, xcd_bands;
+  int tiles_x, tiles_y;
   int stage;
   const double* Uin;
   const double* Un;
@@ -53,6 +53,7 @@ struct StageArgs {
   // tile for the learned indicator ([e*3 + k], cell_means_rpa with w0), or null
   double* means;
   const double* __restrict__ w0;
+  const double* __restrict__ tensor;  // 2D p=2: 1D tables of vol_tensor_wave
   double* uavg;   // with means: also the sensor's cell averages [e*5 + f] (sensor_nodal_mean), or null
   double* psens;  // with uavg: their sensor pressures [e]
   const int* gate;  // set and nonzero: the launch does nothing (a step skipped by the device-side time control)
@@ -214,81 +215,51 @@ __device__ inline int halo_source(int h, int ex0, int ey0, const StageArgs& a, i
   }
 }
 
-#ifndef DGX_STAGE_PAD
-#define DGX_STAGE_PAD 1  // pad per-element LDS strides against bank conflicts
-#endif
-#ifndef DGX_STAGE_MFMA64
-#define DGX_STAGE_MFMA64 1  // 2D p=2 FP64 element phases on the matrix cores (0: VALU batches)
-#endif
-#ifndef DGX_STAGE_PERSIST
-#define DGX_STAGE_PERSIST 0  // 1: persistent blocks, next tile loaded during the current one
-#endif
-
 // Per-element LDS stride for n doubles: with padding, the smallest stride
 // >= n whose element starts fall on distinct, non-overlapping 16-byte bank
 // groups for the four elements a wave reads at once (2*stride mod 32 dwords
 // in [4, 28]).
 constexpr bool bank_ok(int n) { return (2 * n) % 32 >= 4 && (2 * n) % 32 <= 28; }
-constexpr int lds_stride(int n) { return !DGX_STAGE_PAD || bank_ok(n) ? n : lds_stride(n + 1); }
+constexpr int lds_stride(int n) { return bank_ok(n) ? n : lds_stride(n + 1); }
 
-// Tile origin of the i-th tile a block processes.  Blocks are dispatched
-// round-robin over the 8 XCDs; with XCD bands the tiles of each XCD form a
-// contiguous band of the grid so that halo rows are shared in its L2.
-__device__ inline int tile_of(const StageArgs& a, int i) {
-  const int ntiles = a.tiles_x * a.tiles_y;
-  if (a.xcd_bands) {
-    const int per = ntiles >> 3, nbx = gridDim.x >> 3;
-    const int x = blockIdx.x & 7, j = (blockIdx.x >> 3) + i * nbx;
-    return j < per ? x * per + j : -1;
-  }
-  const int t = blockIdx.x + i * gridDim.x;
-  return t < ntiles ? t : -1;
+// The tile of this block, or -1.  Blocks are dispatched round-robin over the
+// 8 XCDs; the tiles of each XCD form a contiguous band of the grid, so that
+// halo rows are shared in its L2 (the launch has a multiple of 8 blocks).
+__device__ inline int tile_of(const StageArgs& a) {
+  const int per = gridDim.x >> 3, t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  return t < a.tiles_x * a.tiles_y ? t : -1;
 }
 
-// RAG (2D, no persistent grid): the grid's sides need not be whole tiles; the
-// tile's elements past its ends repeat the tile's first element and are not
-// stored.
-// VEC: the tile state, the RK operands and the stage output move as 16-byte
-// pairs (tile rows are contiguous in HBM and in LDS; every state pointer and
-// row start is 16-byte aligned and, with RAG, every row of a tile a whole
-// number of pairs, which the host checks before it picks this instance).
-template <int D, int P, int PH, int FL, int MODE, int TX, int TY, int PREC, bool VEC = false, bool RAG = false>
+// The tile kernel with the element phases as batches on the vector units: 1D,
+// and first order in 2D (four nodes and points per element: no matrix shape).
+// RAG (2D): the grid's sides need not be whole tiles; the tile's elements past
+// its ends repeat the tile's first element and are not stored.
+template <int D, int P, int PH, int FL, int MODE, int TX, int TY, bool RAG>
 __global__ __launch_bounds__(256) void k_stage(StageArgs a) {
   if (a.gate && *a.gate) return;
-  static_assert(!RAG || (D == 2 && !DGX_STAGE_PERSIST), "ragged tiles: 2D");
+  static_assert(!RAG || D == 2, "ragged tiles: 2D");
   using V = Vol<D, P, PH>;
   using T = Tile<D, TX, TY>;
   constexpr int NF = V::NF, Ns = V::Ns, NG = V::NG, Ms = V::Ms, MG = Shape<D, P>::MG;
   constexpr int NU = V::NU, NQE = V::NQE, NQ = V::NQ, TPE = V::TPE, EPB = V::EPB;
   constexpr int NT = T::NT, NFACE = T::NFACE, NH = T::NH, HT = NF * Ms;
   constexpr int SU = lds_stride(NU), SQ = lds_stride(NQE), SW = lds_stride(NG * NQ);
-  // element phases on the matrix cores (FP64, or FP32 in the mixed-precision mode) or as VALU batches
-  // PREC 0: FP64; 1: FP32 contractions; 2: split-BF16 contractions with FP32 accumulation
-  constexpr bool MFW = D == 2 && P == 2 && NT % 16 == 0 && PH <= 1 && (PREC >= 1 || DGX_STAGE_MFMA64);
-  using TW = typename std::conditional<PREC >= 1, float, double>::type;
   constexpr int NNC = V::NNC;    // non-conservative fields: the last NNC
   constexpr int NWP = NF + NNC;  // per face point: F, and the non-conservative terms
-  constexpr int NW_FACE = NFACE * MG * NWP, NW_VOL = MFW ? 0 : EPB * SW;
-  constexpr int NW_MF = MFW ? 4 * vol_wave_lds<TW, PH>() : 0;
-  constexpr int NW0 = NW_FACE > NW_VOL ? NW_FACE : NW_VOL;
-  constexpr int NW = NW0 > NW_MF ? NW0 : NW_MF;
+  constexpr int NW_FACE = NFACE * MG * NWP, NW_VOL = EPB * SW;
+  constexpr int NW = NW_FACE > NW_VOL ? NW_FACE : NW_VOL;
   constexpr int NGEO = 1 + D * D;
-  static_assert(PREC == 0 || MFW, "mixed precision: 2D p=2 tiles of a multiple of 16 elements");
-  __shared__ int sNodeQ[18];
-  // per-thread counts of the loaded quantities (state entries in groups of VW)
-  static_assert(!VEC || (D == 2 && SU == NU && (TX * NU) % 2 == 0), "paired state rows");
-  constexpr int VW = VEC ? 2 : 1;
-  constexpr int R_UV = (NT * NU / VW + 255) / 256, R_U = R_UV * VW;
-  constexpr int R_H = (NH * HT + 255) / 256;
+  // per-thread counts of the loaded quantities
+  constexpr int R_U = (NT * NU + 255) / 256, R_H = (NH * HT + 255) / 256;
   constexpr int R_G = (NT * NGEO + 255) / 256, R_F = (NFACE * 4 + 255) / 256;
 
-  __shared__ __align__(16) double sU[NT * SU];
+  __shared__ double sU[NT * SU];
   __shared__ double sH[NH * HT];
   __shared__ double sQ[NT * SQ];
   __shared__ double sW[NW];  // face-point fluxes, then per-point volume values
   __shared__ double sPhi[V::NTAB_PHI];
   __shared__ double sDphi[PH ? V::NTAB_D : 1];
-  __shared__ double sDw[MFW ? 1 : V::NTAB_D];  // the matrix-core path keeps its operand in registers
+  __shared__ double sDw[V::NTAB_D];
   __shared__ double sPw[PH ? V::NTAB_PHI : 1];
   __shared__ double sMinv[Ns * Ns];
   __shared__ double sPsi[MG * Ms], sPsiw[MG * Ms];
@@ -300,371 +271,699 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs a) {
   static_assert(NT <= 128 && NH <= 128, "face sources fit 8 bits");
   const VolTables<D, P, PH> tb{sPhi, sDphi, sDw, sPw, sMinv};
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, tile = tile_of(a);
+  if (tile < 0) return;
   const bool shared_minv = a.minv_stride == 0;
-  // reference tables and the first tile's inputs are fetched together (one wait)
+  // reference tables and the tile's inputs are fetched together (one wait)
   static_assert(MG * Ms <= 256, "face tables fit one pass");
-  VolTableFetch<D, P, PH, !MFW> tf;
+  VolTableFetch<D, P, PH, true> tf;
   tf.fetch(a.phi, a.dphi, a.phi_w, a.dphi_w, a.Minv, MODE == 1 && shared_minv, tid);
   double psi_r = 0.0, psiw_r = 0.0;
   if (tid < MG * Ms) { psi_r = a.psi[tid]; psiw_r = a.psi_w[tid]; }
-  if constexpr (MFW) node_q_table<NF>(sNodeQ, tid);
   const double dt = (MODE == 1) ? a.dt[0] : 0.0;
-
-  // registers holding the next tile's inputs while the current one computes
+  const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
   double pu[R_U], ph[R_H], pg[R_G], pf[R_F];
-  auto issue = [&](int tile) {
-    const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
 #pragma unroll
-    for (int r = 0; r < R_UV; ++r) {
-      const int k = VW * (tid + r * 256);
-      if (k < NT * NU) {
-        const int ty = k / (TX * NU);
-        const double* src = a.Uin + ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
-        if constexpr (RAG) {
-          if (ey0 + ty >= a.ny || k - ty * TX * NU >= (a.nx - ex0) * NU)
-            src = a.Uin + ((size_t)ey0 * a.nx + ex0) * NU + (VEC && NU % 2 ? k % (NU - 1) : k % NU);
-        }
-        if constexpr (VEC) {
-          const double2 v = *reinterpret_cast<const double2*>(src);
-          pu[2 * r] = v.x;
-          pu[2 * r + 1] = v.y;
-        } else {
-          pu[r] = *src;
-        }
+  for (int r = 0; r < R_U; ++r) {
+    const int k = tid + r * 256;
+    if (k < NT * NU) {
+      const int ty = k / (TX * NU);
+      const double* src = a.Uin + ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
+      if constexpr (RAG) {
+        if (ey0 + ty >= a.ny || k - ty * TX * NU >= (a.nx - ex0) * NU)
+          src = a.Uin + ((size_t)ey0 * a.nx + ex0) * NU + k % NU;
       }
+      pu[r] = *src;
     }
+  }
 #pragma unroll
-    for (int r = 0; r < R_H; ++r) {
-      const int k = tid + r * 256;
-      if (k < NH * HT) {
-        const int h = k / HT, q = k % HT, f = q / Ms, j = q % Ms;
-        int cl = 0;
-        const int e = halo_source<D, TX, TY, RAG>(h, ex0, ey0, a, cl);
-        ph[r] = (e >= 0) ? a.Uin[((size_t)e * NF + f) * Ns + closure_node<D, P>(cl, j)] : 0.0;
+  for (int r = 0; r < R_H; ++r) {
+    const int k = tid + r * 256;
+    if (k < NH * HT) {
+      const int h = k / HT, q = k % HT, f = q / Ms, j = q % Ms;
+      int cl = 0;
+      const int e = halo_source<D, TX, TY, RAG>(h, ex0, ey0, a, cl);
+      ph[r] = (e >= 0) ? a.Uin[((size_t)e * NF + f) * Ns + closure_node<D, P>(cl, j)] : 0.0;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R_G; ++r) {
+    const int k = tid + r * 256;
+    if (k < NT * NGEO) {
+      const int el = k / NGEO, q = k % NGEO;
+      const int ty = RAG ? min(el / TX, a.ny - 1 - ey0) : el / TX, tx = RAG ? min(el % TX, a.nx - 1 - ex0) : el % TX;
+      const int eg = ((ey0 + ty) * a.nx + ex0 + tx) * a.geo_stride;
+      pg[r] = q == 0 ? a.J[eg] : a.invJac[eg * D * D + q - 1];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R_F; ++r) {
+    const int k = tid + r * 256;
+    if (k < NFACE * 4) {
+      const int fi = k / 4, q = k % 4;
+      const double* src;
+      if (D == 1 || fi < T::NFX) {
+        int ty = (D == 1) ? 0 : fi / (TX + 1), fx = (D == 1) ? fi : fi % (TX + 1);
+        if constexpr (RAG) ty = min(ty, a.ny - 1 - ey0), fx = min(fx, a.nx - ex0);
+        src = a.gx + ((size_t)(ey0 + ty) * (a.nx + 1) + ex0 + fx) * 4;
+      } else {
+        const int fj = fi - T::NFX;
+        int fy = fj / TX, tx = fj % TX;
+        if constexpr (RAG) fy = min(fy, a.ny - ey0), tx = min(tx, a.nx - 1 - ex0);
+        src = a.gy + ((size_t)(ey0 + fy) * a.nx + ex0 + tx) * 4;
       }
+      pf[r] = src[q];
     }
-#pragma unroll
-    for (int r = 0; r < R_G; ++r) {
-      const int k = tid + r * 256;
-      if (k < NT * NGEO) {
-        const int el = k / NGEO, q = k % NGEO;
-        const int ty = RAG ? min(el / TX, a.ny - 1 - ey0) : el / TX, tx = RAG ? min(el % TX, a.nx - 1 - ex0) : el % TX;
-        const int eg = ((ey0 + ty) * a.nx + ex0 + tx) * a.geo_stride;
-        pg[r] = q == 0 ? a.J[eg] : a.invJac[eg * D * D + q - 1];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R_F; ++r) {
-      const int k = tid + r * 256;
-      if (k < NFACE * 4) {
-        const int fi = k / 4, q = k % 4;
-        const double* src;
-        if (D == 1 || fi < T::NFX) {
-          int ty = (D == 1) ? 0 : fi / (TX + 1), fx = (D == 1) ? fi : fi % (TX + 1);
-          if constexpr (RAG) ty = min(ty, a.ny - 1 - ey0), fx = min(fx, a.nx - ex0);
-          src = a.gx + ((size_t)(ey0 + ty) * (a.nx + 1) + ex0 + fx) * 4;
-        } else {
-          const int fj = fi - T::NFX;
-          int fy = fj / TX, tx = fj % TX;
-          if constexpr (RAG) fy = min(fy, a.ny - ey0), tx = min(tx, a.nx - 1 - ex0);
-          src = a.gy + ((size_t)(ey0 + fy) * a.nx + ex0 + tx) * 4;
-        }
-        pf[r] = src[q];
-      }
-    }
-  };
-  auto commit = [&]() {
-#pragma unroll
-    for (int r = 0; r < R_UV; ++r) {
-      const int k = VW * (tid + r * 256);
-      if (k < NT * NU) {
-        if constexpr (VEC)
-          *reinterpret_cast<double2*>(sU + k) = make_double2(pu[2 * r], pu[2 * r + 1]);  // SU == NU
-        else
-          sU[(k / NU) * SU + k % NU] = pu[r];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R_H; ++r) {
-      const int k = tid + r * 256;
-      if (k < NH * HT) sH[k] = ph[r];
-    }
-#pragma unroll
-    for (int r = 0; r < R_G; ++r) {
-      const int k = tid + r * 256;
-      if (k < NT * NGEO) sGeo[k] = pg[r];
-    }
-#pragma unroll
-    for (int r = 0; r < R_F; ++r) {
-      const int k = tid + r * 256;
-      if (k < NFACE * 4) sFG[k] = pf[r];
-    }
-  };
-
+  }
   // the descriptor of every tile face, once per face (one lane each, while
   // the tile's loads are in flight); the face and integration phases read it
-  auto descs = [&](int tile) {
-    const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
-    for (int fi = tid; fi < NFACE; fi += 256) {
-      const FaceDesc fd = face_desc<D, TX, TY, RAG>(fi, ex0, ey0, a);
-      sFD[fi] = ((fd.dst[0] + 1) | (fd.edge[0] << 8) | (fd.cl[0] << 10)) |
-                (((fd.dst[1] + 1) | (fd.edge[1] << 8) | (fd.cl[1] << 10)) << 16);
-      sFS[fi] = (fd.src[0] + 128) | ((fd.src[1] + 128) << 8) | (fd.tag << 16);
-    }
-  };
-  int tile = tile_of(a, 0);
-  if (tile >= 0) {
-    issue(tile);
-    descs(tile);
+  for (int fi = tid; fi < NFACE; fi += 256) {
+    const FaceDesc fd = face_desc<D, TX, TY, RAG>(fi, ex0, ey0, a);
+    sFD[fi] = ((fd.dst[0] + 1) | (fd.edge[0] << 8) | (fd.cl[0] << 10)) |
+              (((fd.dst[1] + 1) | (fd.edge[1] << 8) | (fd.cl[1] << 10)) << 16);
+    sFS[fi] = (fd.src[0] + 128) | ((fd.src[1] + 128) << 8) | (fd.tag << 16);
   }
   tf.store(tb, MODE == 1 && shared_minv, tid);
   if (tid < MG * Ms) { sPsi[tid] = psi_r; sPsiw[tid] = psiw_r; }
-  for (int it = 0; tile >= 0; ++it) {
-    const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
-    auto gidx = [&](int k) -> size_t {
-      const int ty = k / (TX * NU);
-      return ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
-    };
-    auto in_grid = [&](int k) {  // tile entry k belongs to the grid (its row's end is a whole number of elements)
-      const int ty = k / (TX * NU);
-      return !RAG || (ey0 + ty < a.ny && k - ty * TX * NU < (a.nx - ex0) * NU);
-    };
-    commit();
-    if (it > 0) descs(tile);  // the previous tile's descriptors were read up to its last barrier
-    __syncthreads();
-    // the output's Dt factor once per element (read after several barriers)
-    if (MODE == 1 && tid < NT) sDte[tid] = shared_minv ? dt * (a.J0 / sGeo[tid * NGEO]) : dt;
-    // RK operands of this thread's output entries, then the next tile's
-    // inputs: all in flight during the compute below
-    double pre_un[R_U], pre_acc[R_U];
+  auto gidx = [&](int k) -> size_t {
+    const int ty = k / (TX * NU);
+    return ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
+  };
+  auto in_grid = [&](int k) {  // tile entry k belongs to the grid (its row's end is a whole number of elements)
+    const int ty = k / (TX * NU);
+    return !RAG || (ey0 + ty < a.ny && k - ty * TX * NU < (a.nx - ex0) * NU);
+  };
 #pragma unroll
-    for (int r = 0; r < R_UV; ++r) {
+  for (int r = 0; r < R_U; ++r) {
+    const int k = tid + r * 256;
+    if (k < NT * NU) sU[(k / NU) * SU + k % NU] = pu[r];
+  }
 #pragma unroll
-      for (int v = 0; v < VW; ++v) pre_un[r * VW + v] = pre_acc[r * VW + v] = 0.0;
-      const int k = VW * (tid + r * 256);
-      if (MODE == 1 && k < NT * NU && in_grid(k)) {
-        const size_t i = gidx(k);
-        if constexpr (VEC) {
-          if (a.stage < 3) {
-            const double2 v = *reinterpret_cast<const double2*>(a.Un + i);
-            pre_un[2 * r] = v.x;
-            pre_un[2 * r + 1] = v.y;
-          }
-          if (a.stage > 0) {
-            const double2 v = *reinterpret_cast<const double2*>(a.Uacc + i);
-            pre_acc[2 * r] = v.x;
-            pre_acc[2 * r + 1] = v.y;
-          }
-        } else {
-          if (a.stage < 3) pre_un[r] = a.Un[i];
-          if (a.stage > 0) pre_acc[r] = a.Uacc[i];
-        }
-      }
+  for (int r = 0; r < R_H; ++r) {
+    const int k = tid + r * 256;
+    if (k < NH * HT) sH[k] = ph[r];
+  }
+#pragma unroll
+  for (int r = 0; r < R_G; ++r) {
+    const int k = tid + r * 256;
+    if (k < NT * NGEO) sGeo[k] = pg[r];
+  }
+#pragma unroll
+  for (int r = 0; r < R_F; ++r) {
+    const int k = tid + r * 256;
+    if (k < NFACE * 4) sFG[k] = pf[r];
+  }
+  __syncthreads();
+  // the output's Dt factor once per element (read after several barriers)
+  if (MODE == 1 && tid < NT) sDte[tid] = shared_minv ? dt * (a.J0 / sGeo[tid * NGEO]) : dt;
+  // RK operands of this thread's output entries, in flight during the compute below
+  double pre_un[R_U], pre_acc[R_U];
+#pragma unroll
+  for (int r = 0; r < R_U; ++r) {
+    pre_un[r] = pre_acc[r] = 0.0;
+    const int k = tid + r * 256;
+    if (MODE == 1 && k < NT * NU && in_grid(k)) {
+      const size_t i = gidx(k);
+      if (a.stage < 3) pre_un[r] = a.Un[i];
+      if (a.stage > 0) pre_acc[r] = a.Uacc[i];
     }
-    const int next = DGX_STAGE_PERSIST ? tile_of(a, it + 1) : -1;
+  }
 
-    // ---- faces: one lane per (face, Gauss point)
-    for (int itf = tid; itf < NFACE * MG; itf += 256) {
-      const int fi = itf / MG, g = itf % MG;
-      // descriptor: per side (dst + 1) | edge << 8 | cl << 10 in sFD, source slot + 128 in sFS
-      const int fdw = sFD[fi], fsw = sFS[fi];
-      const int fsrc[2] = {(fsw & 255) - 128, ((fsw >> 8) & 255) - 128};
-      const int fcl[2] = {(fdw >> 10) & 7, (fdw >> 26) & 7};
-      const int ftag = fsw >> 16;
-      const double* fg = sFG + fi * 4;
-      const double nxv = fg[0], nyv = (D == 2) ? fg[1] : 0.0, jf0 = fg[2], jf1 = fg[3];
-      double tr[2][NF][Ms];
+  // ---- faces: one lane per (face, Gauss point)
+  for (int itf = tid; itf < NFACE * MG; itf += 256) {
+    const int fi = itf / MG, g = itf % MG;
+    // descriptor: per side (dst + 1) | edge << 8 | cl << 10 in sFD, source slot + 128 in sFS
+    const int fdw = sFD[fi], fsw = sFS[fi];
+    const int fsrc[2] = {(fsw & 255) - 128, ((fsw >> 8) & 255) - 128};
+    const int fcl[2] = {(fdw >> 10) & 7, (fdw >> 26) & 7};
+    const int ftag = fsw >> 16;
+    const double* fg = sFG + fi * 4;
+    const double nxv = fg[0], nyv = (D == 2) ? fg[1] : 0.0, jf0 = fg[2], jf1 = fg[3];
+    double tr[2][NF][Ms];
 #pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const int s = fsrc[d];
+    for (int d = 0; d < 2; ++d) {
+      const int s = fsrc[d];
 #pragma unroll
-        for (int j = 0; j < Ms; ++j) {
-          if (s >= 0) {
-            const int node = closure_node<D, P>(fcl[d], j);
+      for (int j = 0; j < Ms; ++j) {
+        if (s >= 0) {
+          const int node = closure_node<D, P>(fcl[d], j);
 #pragma unroll
-            for (int f = 0; f < NF; ++f) tr[d][f][j] = sU[s * SU + f * Ns + node];
-          } else {
+          for (int f = 0; f < NF; ++f) tr[d][f][j] = sU[s * SU + f * Ns + node];
+        } else {
 #pragma unroll
-            for (int f = 0; f < NF; ++f) tr[d][f][j] = sH[(-1 - s) * HT + f * Ms + j];
-          }
+          for (int f = 0; f < NF; ++f) tr[d][f][j] = sH[(-1 - s) * HT + f * Ms + j];
         }
       }
-      if (ftag == BC_REFLECTIVE) {  // boundaries.cu:20-67 on the nodal face values
+    }
+    if (ftag == BC_REFLECTIVE) {  // boundaries.cu:20-67 on the nodal face values
 #pragma unroll
-        for (int j = 0; j < Ms; ++j) {
-          if constexpr (D == 1) {
-            tr[1][1][j] = -tr[1][1][j];
-          } else {
-            const double nx2 = nxv * nxv, ny2 = nyv * nyv, m2nxny = -2 * nxv * nyv;
-            const double inv = 1.0 / (nx2 + ny2);
-            const double vxL = tr[0][1][j], vyL = tr[0][2][j];
-            tr[1][1][j] = inv * ((-nx2 + ny2) * vxL + m2nxny * vyL);
-            tr[1][2][j] = inv * (m2nxny * vxL + (nx2 - ny2) * vyL);
-          }
+      for (int j = 0; j < Ms; ++j) {
+        if constexpr (D == 1) {
+          tr[1][1][j] = -tr[1][1][j];
+        } else {
+          const double nx2 = nxv * nxv, ny2 = nyv * nyv, m2nxny = -2 * nxv * nyv;
+          const double inv = 1.0 / (nx2 + ny2);
+          const double vxL = tr[0][1][j], vyL = tr[0][2][j];
+          tr[1][1][j] = inv * ((-nx2 + ny2) * vxL + m2nxny * vyL);
+          tr[1][2][j] = inv * (m2nxny * vxL + (nx2 - ny2) * vyL);
         }
       }
-      double ul[NF], ur[NF], F[NF], nc[NF];
+    }
+    double ul[NF], ur[NF], F[NF], nc[NF];
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        double sl = 0.0, sr = 0.0;
+    for (int f = 0; f < NF; ++f) {
+      double sl = 0.0, sr = 0.0;
 #pragma unroll
-        for (int j = 0; j < Ms; ++j) {
-          sl += tr[0][f][j] * sPsi[g + j * MG];
-          sr += tr[1][f][j] * sPsi[g + j * MG];
-        }
-        ul[f] = sl;
-        ur[f] = sr;
+      for (int j = 0; j < Ms; ++j) {
+        sl += tr[0][f][j] * sPsi[g + j * MG];
+        sr += tr[1][f][j] * sPsi[g + j * MG];
       }
-      riemann<D, PH, FL>(ul, ur, nxv, nyv, F, nc);
-      // the non-conservative terms are zero except for the last NNC fields
-      // (alpha; phinc; alpha and beta): keep F and those; sides and face
-      // Jacobians at integration
-      double* w = sW + (fi * MG + g) * NWP;
+      ul[f] = sl;
+      ur[f] = sr;
+    }
+    riemann<D, PH, FL>(ul, ur, nxv, nyv, F, nc);
+    // the non-conservative terms are zero except for the last NNC fields
+    // (alpha; phinc; alpha and beta): keep F and those; sides and face
+    // Jacobians at integration
+    double* w = sW + (fi * MG + g) * NWP;
 #pragma unroll
-      for (int f = 0; f < NF; ++f) w[f] = F[f];
+    for (int f = 0; f < NF; ++f) w[f] = F[f];
 #pragma unroll
-      for (int m = 0; m < NNC; ++m) w[NF + m] = nc[NF - NNC + m];
+    for (int m = 0; m < NNC; ++m) w[NF + m] = nc[NF - NNC + m];
+  }
+  __syncthreads();
+  // ---- face integration against psi_w into the receiving elements' slots
+  for (int itf = tid; itf < NFACE * 2 * Ms; itf += 256) {
+    const int fi = itf / (2 * Ms), d = (itf / Ms) % 2, j = itf % Ms;
+    const int side = (sFD[fi] >> (16 * d)) & 0xffff;
+    const int dst = (side & 0xff) - 1;
+    if (dst < 0) continue;
+    const int cl = side >> 10, edge = (side >> 8) & 3;
+    const int jf = (D == 2 && cl >= 4) ? reversed_pos<P>(j) : j;
+    double* q = sQ + dst * SQ + edge * NF * Ms;
+    const double jfd = sFG[fi * 4 + 2 + d];
+    // the side's sign: fma(-1, F, nc) is -F + nc rounded once, the same
+    // bits as the sum, without computing both sums and selecting per lane
+    const double sgn = d ? 1.0 : -1.0;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      double s = 0.0;
+#pragma unroll
+      for (int g = 0; g < MG; ++g) {
+        const double* w = sW + (fi * MG + g) * NWP;
+        const double ncf = f >= NF - NNC ? w[NF + f - (NF - NNC)] : 0.0;
+        // q_L = (-F + nc) JF_0, q_R = (F + nc) JF_1 (physics.cu:800-804, kernels.cu:199-228)
+        const double qv = __builtin_fma(sgn, w[f], ncf) * jfd;
+        s += sPsiw[g + j * MG] * qv;
+      }
+      q[f * Ms + jf] = s;
+    }
+  }
+  __syncthreads();
+
+  // ---- element phases
+  for (int b = 0; b < NT; b += EPB) {
+    {
+      const int el = b + tid / TPE, g = tid % TPE;
+      if (el < NT && g < NG)
+        vol_phase1<D, P, PH>(tb, g, sU + el * SU, sGeo[el * NGEO], sGeo + el * NGEO + 1,
+                             sW + (el - b) * SW + g * NQ);
     }
     __syncthreads();
-    // the next tile's inputs (persistent blocks): in flight from here to the
-    // next commit, past the face phase, whose registers peak
-    if (next >= 0) issue(next);
-    // ---- face integration against psi_w into the receiving elements' slots
-    for (int itf = tid; itf < NFACE * 2 * Ms; itf += 256) {
-      const int fi = itf / (2 * Ms), d = (itf / Ms) % 2, j = itf % Ms;
-      const int side = (sFD[fi] >> (16 * d)) & 0xffff;
-      const int dst = (side & 0xff) - 1;
-      if (dst < 0) continue;
-      const int cl = side >> 10, edge = (side >> 8) & 3;
-      const int jf = (D == 2 && cl >= 4) ? reversed_pos<P>(j) : j;
-      double* q = sQ + dst * SQ + edge * NF * Ms;
-      const double jfd = sFG[fi * 4 + 2 + d];
-      // the side's sign: fma(-1, F, nc) is -F + nc rounded once, the same
-      // bits as the sum, without computing both sums and selecting per lane
-      const double sgn = d ? 1.0 : -1.0;
+    {
+      const int el = b + tid / TPE, i = tid % TPE;
+      double rhs[NF];
+      const bool act = el < NT && i < Ns;
+      if (act) vol_phase2<D, P, PH>(tb, i, sW + (el - b) * SW, sQ + el * SQ, rhs);
+      __syncthreads();
+      if (act)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) sU[el * SU + f * Ns + i] = rhs[f];
+    }
+    __syncthreads();
+  }
+
+  // ---- stage output (coalesced along the tile rows)
+#pragma unroll
+  for (int r = 0; r < R_U; ++r) {
+    const int k = tid + r * 256;
+    if (k >= NT * NU) break;
+    if (!in_grid(k)) continue;
+    const size_t gi = gidx(k);
+    const int el = k / NU, rr = k % NU;
+    if constexpr (MODE == 0) {
+      a.fout[gi] = sU[el * SU + rr];
+    } else {
+      // shared Minv: Minv_e = Minv_0 * J_0 / J_e (affine elements); else per element
+      const double dte = sDte[el];
+      const double* M = shared_minv ? tb.minv : a.Minv + ((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * Ns * Ns;
+      const int f = rr / Ns, i = rr % Ns;
+      const double* R = sU + el * SU + f * Ns;
+      double sol = 0.0;
+#pragma unroll
+      for (int ii = 0; ii < Ns; ++ii) sol += M[ii * Ns + i] * R[ii];
+      rk_combine(a.stage, dte * sol, pre_un[r], pre_acc[r], a.Uacc + gi, a.Uout + gi);
+    }
+  }
+}
+
+// Where the lane of node c of a 2D element (order P) takes its face sums
+// from: the at most two edges whose closure holds the node, and its place
+// there (closure_node), or -1.
+template <int P>
+__device__ inline void node_edges(int c, int* edge, int* pos) {
+  edge[0] = edge[1] = -1;
+  pos[0] = pos[1] = 0;
+  if (c < 0) return;
+  if (c < 4) {  // corner c: first node of edge c, second of the edge before it
+    edge[0] = c;
+    edge[1] = (c + 3) & 3;
+    pos[1] = 1;
+  } else if (c < 4 * P) {
+    edge[0] = (c - 4) / (P - 1);
+    pos[0] = 2 + (c - 4) % (P - 1);
+  }
+}
+
+// The tile kernel for 2D orders 2 and 3, 8 x 4 elements, element phases on the
+// matrix cores (vol_mfma_wave).  Phases: the tile's state, halo traces and
+// geometry into LDS; face fluxes at the Gauss points, one lane each; element
+// phases by wave, whose face sums take the fluxes of an element's four faces
+// straight from there; the RK4 combination.  Two block barriers between the
+// loads and the output.
+//
+// Bound by HBM and by how much of a block's serial chain the other blocks of
+// its CU hide.  1024x512 two-fluid, p = 2: 212 us a launch (755 MB of states,
+// 925 MB measured: 4.4 TB/s of the 4.9 a copy reaches) against 309 us of the
+// kernel before it, which summed the faces into per-element edges behind a
+// barrier of its own, kept the reference tables in LDS (50.8 KB, three blocks
+// a CU; now 30.5 KB and four) and ran 28 16x16x4 products and the fields after
+// E on the vector units; 512x512 single fluid 88 against 121 us; 512x256
+// stiffened 79 against 147 us and p = 3 two-fluid 138 against 489 us, both
+// element phases on the vector units before.  On the way: the RK operands
+// fetched before the face phase, and copied where a stage needs only one,
+// made every wave wait for them there (3.6k of its 36k cycles), the operands
+// of the matrix products read from global memory behind them 4.7k.
+//
+// PREC: 0 FP64, 1 FP32 and 2 split-BF16 contractions of rho, momenta and E
+// (p = 2).  VEC: the tile state, the RK operands and the stage output move as
+// 16-byte pairs (every state pointer and row start is 16-byte aligned and,
+// with RAG, every row of a tile a whole number of pairs, which the host checks
+// before it picks this instance).  RAG: the grid's sides need not be whole
+// tiles; the tile's elements past its ends repeat the tile's first element and
+// are not stored.
+// Waves per SIMD the registers must allow.  Measured, us a step without
+// limiter: p = 2 single fluid 512x512 353 with 4 and 5, 473 with 6 (spills);
+// two-fluid 1024x512 849 with 3 and 4, 917 with 5; stiffened 512x256 315 with 3
+// and 4, 323 with 2; p = 3 single fluid 256x256 202-206 with 2 to 4, two-fluid
+// 512x256 554 with 2, 562 with 3.
+constexpr int stage_waves(int P, int PH) { return P == 2 ? (PH <= 1 ? 4 : 3) : (PH == 0 ? 3 : (PH == 1 ? 2 : 1)); }
+
+template <int P, int PH, int FL, int MODE, int PREC, bool VEC, bool RAG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves(P, PH)))) void k_stage_mfma(StageArgs a) {
+  if (a.gate && *a.gate) return;
+  constexpr int D = 2, TX = 8, TY = 4;
+  using V = Vol<D, P, PH>;
+  using T = Tile<D, TX, TY>;
+  using TW = typename std::conditional<PREC >= 1, float, double>::type;
+  constexpr int NF = V::NF, Ns = V::Ns, Ms = V::Ms, MG = Shape<D, P>::MG, NU = V::NU, NNC = V::NNC;
+  constexpr int NT = T::NT, NFACE = T::NFACE, NFX = T::NFX, NH = T::NH, HT = NF * Ms;
+  constexpr int SU = lds_stride(NU);
+  constexpr int NWP = NF + NNC;  // per face point: F, and the non-conservative terms
+  // P = 2 in FP64: 4x4 products in registers (vol_tensor_wave); else 16x16 ones (vol_mfma_wave)
+  constexpr bool TENSOR = P == 2 && PREC == 0;
+  constexpr int NXT = TENSOR ? 0 : 4 * vol_wave_extra<P, PH>(), NZ = NH * HT > NXT ? NH * HT : NXT;
+  constexpr int VW = VEC ? 2 : 1;
+  static_assert(!VEC || ((TX * NU) % 2 == 0 && (SU == NU || (NU % 2 == 0 && SU % 2 == 0))), "paired state rows");
+  constexpr int R_U = (NT * NU / VW + 255) / 256, R_H = (HT + 7) / 8;
+
+  __shared__ __align__(16) double sU[NT * SU + NZ];  // the tile's state; then the halo traces, later the extra rows
+  __shared__ __align__(16) double sW[NFACE * MG * NWP];  // face-point fluxes
+  // TENSOR: the 1D tables; else the reference tables until every wave has taken
+  // its operands, then the element phases' flux rows
+  constexpr int O_DW = V::NTAB_PHI, O_MINV = O_DW + V::NTAB_D, O_DPHI = O_MINV + Ns * Ns,
+                O_PW = O_DPHI + (NNC ? V::NTAB_D : 0), NTAB = O_PW + (NNC ? V::NTAB_PHI : 0);
+  constexpr int NFLUX = 4 * vol_wave_flux<TW, P>(), NFT = NTAB > NFLUX ? NTAB : NFLUX;
+  __shared__ double sFlux[TENSOR ? kTensorTables * 16 : NFT];
+  __shared__ double sPsi[MG * Ms], sPsiw[MG * Ms];
+  __shared__ double sGeo[NT * 4];     // per element: J * invJac
+  __shared__ double sDte[NT];         // per element: Dt (J_0/J_e with the shared Minv)
+  __shared__ __align__(16) double sFG[NFACE * 4];   // per tile face: n_x, n_y, JF side 0, JF side 1
+  // per tile face and side: where its trace starts in sU (12 bits), its nodes'
+  // offsets there (4 bits each), the face's boundary tag
+  __shared__ unsigned sFS[2 * NFACE];
+  static_assert(NT * SU + NH * HT < 4096, "trace starts fit 12 bits");
+  double* sH = sU + NT * SU;
+
+  const int tid = threadIdx.x, tile = tile_of(a);
+  if (tile < 0) return;
+  const bool shared_minv = a.minv_stride == 0;
+  const double dt = (MODE == 1) ? a.dt[0] : 0.0;
+  const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
+  // tile entry k: its offset from the tile's first entry in a state, whether
+  // the grid holds it (its row's end is a whole number of elements), and its
+  // place in LDS
+  const size_t tile0 = ((size_t)ey0 * a.nx + ex0) * NU;
+  const unsigned row = (unsigned)a.nx * NU;
+  auto offset = [&](int k) -> unsigned {
+    const int ty = k / (TX * NU);
+    return ty * row + (k - ty * TX * NU);
+  };
+  auto in_grid = [&](int k) {
+    const int ty = k / (TX * NU);
+    return !RAG || (ey0 + ty < a.ny && k - ty * TX * NU < (a.nx - ex0) * NU);
+  };
+  auto lds_at = [&](int k) { return SU == NU ? k : (k / NU) * SU + k % NU; };
+
+  // ---- every load of the tile in flight at once: the state, consecutive; the
+  // halo traces, 24 slots of 32 lanes, eight entries at a time; per face (the
+  // first lanes) and per element (one wave's) the geometry
+  double pu[R_U * VW], ph[R_H];
+  unsigned off[R_U];
+#pragma unroll
+  for (int r = 0; r < R_U; ++r) {
+    const int k = VW * (tid + r * 256);
+    off[r] = offset(k);
+    if (k < NT * NU) {
+      unsigned o = off[r];
+      if constexpr (RAG) {
+        if (!in_grid(k)) o = VEC && NU % 2 ? k % (NU - 1) : k % NU;
+      }
+      const double* src = a.Uin + tile0 + o;
+      if constexpr (VEC) {
+        const double2 v = *reinterpret_cast<const double2*>(src);
+        pu[2 * r] = v.x;
+        pu[2 * r + 1] = v.y;
+      } else {
+        pu[r] = *src;
+      }
+    }
+  }
+  const int hs = tid & 31, hq = tid >> 5;
+  int hcl = 0;
+  const int he = hs < NH ? halo_source<D, TX, TY, RAG>(hs, ex0, ey0, a, hcl) : -1;
+  unsigned hnodes = 0;
+#pragma unroll
+  for (int j = 0; j < Ms; ++j) hnodes |= (unsigned)closure_node<D, P>(hcl, j) << (4 * j);
+  if (he >= 0) {
+    const double* src = a.Uin + (size_t)he * NU;
+#pragma unroll
+    for (int r = 0; r < R_H; ++r) {
+      const int q = min(hq + 8 * r, HT - 1), f = q / Ms, j = q - f * Ms;
+      ph[r] = src[f * Ns + ((hnodes >> (4 * j)) & 15)];
+    }
+  }
+  double2 pf0, pf1;
+  double pj = 1.0;
+  if (tid < NFACE) {
+    const int fj = tid - NFX;
+    int x, y;
+    if (tid < NFX) {
+      x = tid % (TX + 1), y = tid / (TX + 1);
+      if constexpr (RAG) y = min(y, a.ny - 1 - ey0), x = min(x, a.nx - ex0);
+    } else {
+      x = fj % TX, y = fj / TX;
+      if constexpr (RAG) y = min(y, a.ny - ey0), x = min(x, a.nx - 1 - ex0);
+    }
+    const double* src = tid < NFX ? a.gx + ((size_t)(ey0 + y) * (a.nx + 1) + ex0 + x) * 4
+                                  : a.gy + ((size_t)(ey0 + y) * a.nx + ex0 + x) * 4;
+    pf0 = reinterpret_cast<const double2*>(src)[0];
+    pf1 = reinterpret_cast<const double2*>(src)[1];
+  } else if (tid >= 128 && tid < 128 + NT) {
+    const int el = tid - 128;
+    const int ty = RAG ? min(el / TX, a.ny - 1 - ey0) : el / TX, tx = RAG ? min(el % TX, a.nx - 1 - ex0) : el % TX;
+    const int eg = ((ey0 + ty) * a.nx + ex0 + tx) * a.geo_stride;
+    pj = a.J[eg];
+    pf0 = reinterpret_cast<const double2*>(a.invJac + (size_t)eg * 4)[0];
+    pf1 = reinterpret_cast<const double2*>(a.invJac + (size_t)eg * 4)[1];
+  }
+  static_assert(NFACE <= 128 && NT <= 32, "one lane per face, one wave for the elements");
+  constexpr int R_T = (V::NTAB_PHI + 255) / 256, R_D = (V::NTAB_D + 255) / 256;
+  double tphi[R_T], tdw[R_D], tminv = 0.0, tdphi[R_D], tpw[R_T], tpsi, tpsiw, tten = 0.0;
+  if constexpr (TENSOR) {
+    tten = a.tensor[min(tid, kTensorTables * 16 - 1)];
+  } else {
+#pragma unroll
+  for (int r = 0; r < R_D; ++r) {
+    const int k = min(tid + r * 256, V::NTAB_D - 1);
+    tdw[r] = a.dphi_w[k];
+    if constexpr (NNC > 0) tdphi[r] = a.dphi[k];
+  }
+#pragma unroll
+  for (int r = 0; r < R_T; ++r) {
+    const int k = min(tid + r * 256, V::NTAB_PHI - 1);
+    tphi[r] = a.phi[k];
+    if constexpr (NNC > 0) tpw[r] = a.phi_w[k];
+  }
+  static_assert(Ns * Ns <= 256, "one round");
+  if (MODE == 1 && shared_minv) tminv = a.Minv[min(tid, Ns * Ns - 1)];
+  }
+  tpsi = a.psi[min(tid, MG * Ms - 1)];
+  tpsiw = a.psi_w[min(tid, MG * Ms - 1)];
+  // where each side of every tile face reads its trace, one lane per face
+  if (tid < NFACE) {
+    const FaceDesc fd = face_desc<D, TX, TY, RAG>(tid, ex0, ey0, a);
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int s = fd.src[d];
+      unsigned w = s >= 0 ? s * SU : NT * SU + (-1 - s) * HT;
+#pragma unroll
+      for (int j = 0; j < Ms; ++j) w |= (unsigned)(s >= 0 ? closure_node<D, P>(fd.cl[d], j) : j) << (12 + 4 * j);
+      sFS[2 * tid + d] = w | (unsigned)(fd.tag == BC_REFLECTIVE) << 31;
+    }
+  }
+  static_assert(12 + 4 * Ms <= 31, "a side's word");
+#pragma unroll
+  for (int r = 0; r < R_U; ++r) {
+    const int k = VW * (tid + r * 256);
+    if (k < NT * NU) {
+      if constexpr (VEC)
+        *reinterpret_cast<double2*>(sU + lds_at(k)) = make_double2(pu[2 * r], pu[2 * r + 1]);
+      else
+        sU[lds_at(k)] = pu[r];
+    }
+  }
+  if (he >= 0)
+#pragma unroll
+    for (int r = 0; r < R_H; ++r)
+      if (HT % 8 == 0 || hq + 8 * r < HT) sH[hs * HT + hq + 8 * r] = ph[r];
+  if (tid < NFACE) {
+    reinterpret_cast<double2*>(sFG)[2 * tid] = pf0;
+    reinterpret_cast<double2*>(sFG)[2 * tid + 1] = pf1;
+  } else if (tid >= 128 && tid < 128 + NT) {
+    double* g = sGeo + (tid - 128) * 4;
+    g[0] = pf0.x * pj;
+    g[1] = pf0.y * pj;
+    g[2] = pf1.x * pj;
+    g[3] = pf1.y * pj;
+    if (MODE == 1) sDte[tid - 128] = shared_minv ? (TENSOR ? dt / pj : dt * (a.J0 / pj)) : dt;
+  }
+  if constexpr (TENSOR) {
+    if (tid < kTensorTables * 16) sFlux[tid] = tten;
+  } else {
+#pragma unroll
+  for (int r = 0; r < R_D; ++r)
+    if (tid + r * 256 < V::NTAB_D) {
+      sFlux[O_DW + tid + r * 256] = tdw[r];
+      if constexpr (NNC > 0) sFlux[O_DPHI + tid + r * 256] = tdphi[r];
+    }
+#pragma unroll
+  for (int r = 0; r < R_T; ++r)
+    if (tid + r * 256 < V::NTAB_PHI) {
+      sFlux[tid + r * 256] = tphi[r];
+      if constexpr (NNC > 0) sFlux[O_PW + tid + r * 256] = tpw[r];
+    }
+  if (tid < Ns * Ns) sFlux[O_MINV + tid] = tminv;
+  }
+  if (tid < MG * Ms) {
+    sPsi[tid] = tpsi;
+    sPsiw[tid] = tpsiw;
+  }
+  __syncthreads();
+  // ---- faces: one lane per (face, Gauss point)
+  for (int itf = tid; itf < NFACE * MG; itf += 256) {
+    const int fi = itf / MG, g = itf % MG;
+    double u[2][NF], tr0[Ms];
+    const double nxv = sFG[4 * fi], nyv = sFG[4 * fi + 1];
+    double psi[Ms];
+#pragma unroll
+    for (int j = 0; j < Ms; ++j) psi[j] = sPsi[g + j * MG];
+    bool wall = false;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const unsigned w = sFS[2 * fi + d];
+      const int base = w & 4095, fs = base >= NT * SU ? Ms : Ns;
+      wall = w >> 31;
+      const double* t[Ms];
+#pragma unroll
+      for (int j = 0; j < Ms; ++j) t[j] = sU + base + ((w >> (12 + 4 * j)) & 15);
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         double s = 0.0;
 #pragma unroll
-        for (int g = 0; g < MG; ++g) {
-          const double* w = sW + (fi * MG + g) * NWP;
-          const double ncf = f >= NF - NNC ? w[NF + f - (NF - NNC)] : 0.0;
-          // q_L = (-F + nc) JF_0, q_R = (F + nc) JF_1 (physics.cu:800-804, kernels.cu:199-228)
-          const double qv = __builtin_fma(sgn, w[f], ncf) * jfd;
-          s += sPsiw[g + j * MG] * qv;
-        }
-        q[f * Ms + jf] = s;
+        for (int j = 0; j < Ms; ++j) s += t[j][f * fs] * psi[j];
+        u[d][f] = s;
       }
     }
-    __syncthreads();
-
-    // ---- element phases
-    if constexpr (MFW) {
-      // with the shared Minv the wave also applies Dt * Minv on the matrix cores
-      const bool wave_minv = MODE == 1 && shared_minv;
-      vol_mfma_wave<TW, PH, NT, SU, SQ, NGEO, TW, PREC == 2>(tb, a.dphi_w, sU, sGeo, sQ, sW, sNodeQ, tid,
-                                                             wave_minv ? tb.minv : nullptr, sDte);
-      __syncthreads();
-    } else {
-    for (int b = 0; b < NT; b += EPB) {
-      {
-        const int el = b + tid / TPE, g = tid % TPE;
-        if (el < NT && g < NG)
-          vol_phase1<D, P, PH>(tb, g, sU + el * SU, sGeo[el * NGEO], sGeo + el * NGEO + 1,
-                               sW + (el - b) * SW + g * NQ);
-      }
-      __syncthreads();
-      {
-        const int el = b + tid / TPE, i = tid % TPE;
-        double rhs[NF];
-        const bool act = el < NT && i < Ns;
-        if (act) vol_phase2<D, P, PH>(tb, i, sW + (el - b) * SW, sQ + el * SQ, rhs);
-        __syncthreads();
-        if (act)
-#pragma unroll
-          for (int f = 0; f < NF; ++f) sU[el * SU + f * Ns + i] = rhs[f];
-      }
-      __syncthreads();
+    if (wall) {  // boundaries.cu:20-67 (the reflection is linear: applied at the point instead of at the nodes)
+      const double nx2 = nxv * nxv, ny2 = nyv * nyv, m2nxny = -2 * nxv * nyv;
+      const double inv = 1.0 / (nx2 + ny2);
+      const double vxL = u[0][1], vyL = u[0][2];
+      u[1][1] = inv * ((-nx2 + ny2) * vxL + m2nxny * vyL);
+      u[1][2] = inv * (m2nxny * vxL + (nx2 - ny2) * vyL);
     }
-    }
-
-    // ---- stage output (coalesced along the tile rows, VW entries per step)
+    double F[NF], nc[NF];
+    riemann<D, PH, FL>(u[0], u[1], nxv, nyv, F, nc);
+    // the non-conservative terms are zero except for the last NNC fields
+    double* w = sW + (fi * MG + g) * NWP;
 #pragma unroll
-    for (int r = 0; r < R_UV; ++r) {
-      const int k0 = VW * (tid + r * 256);
-      if (k0 >= NT * NU) break;
-      if (!in_grid(k0)) continue;
-      const size_t gi = gidx(k0);
-      double ov[VW], av[VW];
+    for (int f = 0; f < NF; ++f) w[f] = F[f];
 #pragma unroll
-      for (int v = 0; v < VW; ++v) {
-        const int k = k0 + v, el = k / NU, rr = k % NU;
-        if constexpr (MODE == 0) {
-          ov[v] = sU[el * SU + rr];
-        } else if (MFW && shared_minv) {
-          rk_values(a.stage, sU[el * SU + rr], pre_un[r * VW + v], pre_acc[r * VW + v], av[v], ov[v]);
-          if constexpr (PH == 1) {
-            if (a.means) sU[el * SU + rr] = ov[v];  // this thread's own entry: kept for the cell means below
+    for (int m = 0; m < NNC; ++m) w[NF + m] = nc[NF - NNC + m];
+  }
+  // RK operands of this thread's output entries, in flight during the element
+  // phases: base + beta*du is the stage output, acc + gamma*du the accumulator
+  // (rk_values; stage 0 starts the accumulator from U^n, stage 3 puts out the
+  // accumulator: one operand)
+  double pre_base[R_U * VW], pre_acc[R_U * VW];
+  const bool two = a.stage == 1 || a.stage == 2;
+  if constexpr (MODE == 1) {
+    auto fetch = [&](const double* from, double* to) {
+#pragma unroll
+      for (int r = 0; r < R_U; ++r) {
+        const int k = VW * (tid + r * 256);
+        if (k < NT * NU && in_grid(k)) {
+          if constexpr (VEC) {
+            const double2 v = *reinterpret_cast<const double2*>(from + tile0 + off[r]);
+            to[2 * r] = v.x;
+            to[2 * r + 1] = v.y;
+          } else {
+            to[r] = from[tile0 + off[r]];
           }
-        } else {
-          // shared Minv: Minv_e = Minv_0 * J_0 / J_e (affine elements); else per element
-          const double dte = sDte[el];
-          const double* M = shared_minv ? tb.minv
-                                        : a.Minv + ((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * Ns * Ns;
-          const int f = rr / Ns, i = rr % Ns;
+        }
+      }
+    };
+    fetch(a.stage < 3 ? a.Un : a.Uacc, pre_base);
+    if (two) fetch(a.Uacc, pre_acc);
+  }
+  VolOps<TW, P, PH> op;
+  if constexpr (!TENSOR) op.load(sFlux, sFlux + O_DPHI, sFlux + O_PW, sFlux + O_DW, sFlux + O_MINV, tid);
+  int edge[2], pos[2];
+  node_edges<P>(TENSOR ? tensor_node(tid & 63) : tid & 15, edge, pos);
+  __syncthreads();
+
+  // ---- element phases, with the face terms of node c of element el: the
+  // fluxes of at most two faces against psi_w.  The element is side 0 (the
+  // flux leaves, -F + nc) of its right and upper faces and of the domain's
+  // left and lower ones, else side 1 (F + nc), whose points run backwards
+  // (physics.cu:800-804, kernels.cu:199-228).
+  auto face = [&](int el, double* qs) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) qs[f] = 0.0;
+    const int tx = el % TX, ty = el / TX;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int k = edge[n];
+      if (k < 0) continue;
+      const int fi = (k & 1) ? ty * (TX + 1) + tx + (k == 1) : NFX + (ty + (k == 2)) * TX + tx;
+      const bool side0 = k == 1 || k == 2 || (k == 3 ? ex0 + tx == 0 : ey0 + ty == 0);
+      const int j = side0 ? pos[n] : reversed_pos<P>(pos[n]);
+      const double jf = sFG[4 * fi + (side0 ? 2 : 3)];
+      const double* w = sW + fi * MG * NWP;
+#pragma unroll
+      for (int g = 0; g < MG; ++g) {
+        const double wt = sPsiw[g + j * MG] * jf, ws = side0 ? -wt : wt;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) qs[f] = __builtin_fma(ws, w[g * NWP + f], qs[f]);
+#pragma unroll
+        for (int m = 0; m < NNC; ++m) qs[NF - NNC + m] = __builtin_fma(wt, w[g * NWP + NF + m], qs[NF - NNC + m]);
+      }
+    }
+  };
+  if constexpr (TENSOR)
+    vol_tensor_wave<PH, SU>(sFlux, sU, sGeo, tid, MODE == 1 && shared_minv, sDte, face);
+  else
+    vol_mfma_wave<TW, P, PH, SU, TW, PREC == 2>(op, a.phi, a.dphi_w, sU, sGeo, sFlux, sH, tid,
+                                                MODE == 1 && shared_minv, sDte, face);
+  __syncthreads();
+
+  // ---- stage output (coalesced along the tile rows, VW entries per step)
+  const double gk = MODE == 1 ? kRkGamma[a.stage] : 0.0;
+  const double bk = MODE == 1 ? (a.stage < 3 ? kRkBeta[a.stage + 1] : gk) : 0.0;
+#pragma unroll
+  for (int r = 0; r < R_U; ++r) {
+    const int k0 = VW * (tid + r * 256);
+    if (k0 >= NT * NU) break;
+    if (!in_grid(k0)) continue;
+    double ov[VW], av[VW];
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+      const int at = lds_at(k0) + v;
+      if constexpr (MODE == 0) {
+        ov[v] = sU[at];
+      } else {
+        double du;
+        if (shared_minv) {
+          du = sU[at];
+        } else {  // one Minv per element
+          const int el = (k0 + v) / NU, rr = (k0 + v) % NU, f = rr / Ns, i = rr % Ns;
+          const double* M = a.Minv + ((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * Ns * Ns;
           const double* R = sU + el * SU + f * Ns;
           double sol = 0.0;
 #pragma unroll
           for (int ii = 0; ii < Ns; ++ii) sol += M[ii * Ns + i] * R[ii];
-          rk_values(a.stage, dte * sol, pre_un[r * VW + v], pre_acc[r * VW + v], av[v], ov[v]);
+          du = sDte[el] * sol;
         }
-      }
-      double* out = MODE == 0 ? a.fout + gi : a.Uout + gi;
-      if constexpr (VEC) {
-        *reinterpret_cast<double2*>(out) = make_double2(ov[0], ov[1]);
-        if (MODE == 1 && a.stage < 3) *reinterpret_cast<double2*>(a.Uacc + gi) = make_double2(av[0], av[1]);
-      } else {
-        out[0] = ov[0];
-        if (MODE == 1 && a.stage < 3) a.Uacc[gi] = av[0];
-      }
-    }
-    if constexpr (MODE == 1 && MFW && PH == 1) {
-      if (a.means && shared_minv) {
-        // cell means (cell_means_rpa) and sensor averages (sensor_averages_2d)
-        // of the output tile: one lane per (element, field) forms the field's
-        // two means, then one lane per element the derived values (the same
-        // functions and order as the one-lane forms, so the same bits)
-        static_assert(NW >= 2 * NT * NF, "means staging fits the flux buffer");
-        __syncthreads();  // the output tile is in sU, sW is free
-        double* sM = sW;            // [el*NF + f] mode-0 means
-        double* sA = sW + NT * NF;  // [el*NF + f] sensor nodal means
-        for (int k = tid; k < NT * NF; k += 256) {
-          const int el = k / NF, f = k % NF;
-          if (!in_grid(el * NU)) continue;
-          const double* uf = sU + el * SU + f * Ns;
-          sM[k] = cell_mode0(uf, a.w0);
-          if (a.uavg) {
-            const double v = sensor_nodal_mean<Ns>(uf);
-            sA[k] = v;
-            a.uavg[((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * NF + f] = v;
-          }
-        }
-        __syncthreads();
-        if (tid < NT && in_grid(tid * NU)) {
-          double a3[3];
-          rpa_of_means(sM + tid * NF, a3);
-          const size_t eg = (size_t)(ey0 + tid / TX) * a.nx + ex0 + tid % TX;
-          double* m = a.means + eg * 3;
-          m[0] = a3[0];
-          m[1] = a3[1];
-          m[2] = a3[2];
-          if (a.uavg) a.psens[eg] = sensor_cell<2, 1>(sA + tid * NF, 0).p;
+        av[v] = (two ? pre_acc[r * VW + v] : pre_base[r * VW + v]) + gk * du;
+        ov[v] = pre_base[r * VW + v] + bk * du;
+        if constexpr (P == 2 && PH == 1) {
+          if (a.means) sU[at] = ov[v];  // this thread's own entry: kept for the cell means below
         }
       }
     }
-    if (next >= 0) __syncthreads();  // LDS is refilled for the next tile
-    tile = next;
+    double* out = (MODE == 0 ? a.fout : a.Uout) + tile0 + off[r];
+    double* acc = a.Uacc + tile0 + off[r];
+    if constexpr (VEC) {
+      *reinterpret_cast<double2*>(out) = make_double2(ov[0], ov[1]);
+      if (MODE == 1 && a.stage < 3) *reinterpret_cast<double2*>(acc) = make_double2(av[0], av[1]);
+    } else {
+      out[0] = ov[0];
+      if (MODE == 1 && a.stage < 3) acc[0] = av[0];
+    }
+  }
+  if constexpr (MODE == 1 && P == 2 && PH == 1) {
+    if (a.means && shared_minv) {
+      // cell means (cell_means_rpa) and sensor averages (sensor_averages_2d)
+      // of the output tile: one lane per (element, field) forms the field's
+      // two means, then one lane per element the derived values (the same
+      // functions and order as the one-lane forms, so the same bits)
+      static_assert(NFACE * MG * NWP >= 2 * NT * NF, "means staging fits the flux buffer");
+      __syncthreads();  // the output tile is in sU, sW is free
+      double* sM = sW;            // [el*NF + f] mode-0 means
+      double* sA = sW + NT * NF;  // [el*NF + f] sensor nodal means
+      for (int k = tid; k < NT * NF; k += 256) {
+        const int el = k / NF, f = k % NF;
+        if (!in_grid(el * NU)) continue;
+        const double* uf = sU + el * SU + f * Ns;
+        sM[k] = cell_mode0(uf, a.w0);
+        if (a.uavg) {
+          const double v = sensor_nodal_mean<Ns>(uf);
+          sA[k] = v;
+          a.uavg[((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * NF + f] = v;
+        }
+      }
+      __syncthreads();
+      if (tid < NT && in_grid(tid * NU)) {
+        double a3[3];
+        rpa_of_means(sM + tid * NF, a3);
+        const size_t eg = (size_t)(ey0 + tid / TX) * a.nx + ex0 + tid % TX;
+        double* m = a.means + eg * 3;
+        m[0] = a3[0];
+        m[1] = a3[1];
+        m[2] = a3[2];
+        if (a.uavg) a.psens[eg] = sensor_cell<2, 1>(sA + tid * NF, 0).p;
+      }
+    }
   }
 }
 
@@ -674,14 +973,8 @@ struct TileShape;
 // 1D: 128 elements per tile, or 8 where 128 does not divide the mesh
 template <>
 struct TileShape<1> { static constexpr int TX = 128, TX_SMALL = 8, TY = 1; };
-#ifndef DGX_TILE2_TX
-#define DGX_TILE2_TX 8
-#endif
-#ifndef DGX_TILE2_TY
-#define DGX_TILE2_TY 4
-#endif
 template <>
-struct TileShape<2> { static constexpr int TX = DGX_TILE2_TX, TY = DGX_TILE2_TY; };
+struct TileShape<2> { static constexpr int TX = 8, TY = 4; };
 
 // fn(dim, order, flux) with all three as integral constants
 template <typename Fn>
@@ -722,79 +1015,63 @@ hipError_t launch_stage_phys(const Solver& s, int mode, int stage, const double*
   const int ntiles = a.tiles_x * a.tiles_y;
   a.stage = stage; a.Uin = Uin; a.Un = Un; a.Uacc = Uacc; a.Uout = Uout; a.dt = dt_dev; a.fout = f_out;
   a.gate = s.gate;
+  a.tensor = s.t.tensor;
   a.w0 = s.t.mlp_vinv;  // first row: the mode-0 weights
   return dispatch_stage(s.cfg, [&](auto d, auto p, auto fl) -> hipError_t {
     constexpr int D = decltype(d)::value;
-    auto go = [&](auto txc) -> hipError_t {
-      constexpr int P = decltype(p)::value, FL = decltype(fl)::value;
-      constexpr int TX = decltype(txc)::value, TY = TileShape<D>::TY;
-      auto kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 0> : k_stage<D, P, PH, FL, 1, TX, TY, 0>;
-      if (ragged) {
-        if constexpr (D == 2) {
-          kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 0, false, true>
-                           : k_stage<D, P, PH, FL, 1, TX, TY, 0, false, true>;
-          if constexpr (P == 2 && PH <= 1) {
-            // rows start on pairs, and end on them, when an element is a
-            // whole number of pairs or the grid has an even number of columns
-            constexpr bool even = Vol<D, P, PH>::NU % 2 == 0;
-            auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-            if ((even || c.nx % 2 == 0) && al(Uin) && (mode == 0 ? al(f_out) : al(Un) && al(Uacc) && al(Uout)))
-              kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 0, true, true>
-                               : k_stage<D, P, PH, FL, 1, TX, TY, 0, true, true>;
-          }
-        } else {
-          return hipErrorInvalidValue;  // 1D ragged meshes run the whole-step or the face + element kernels
-        }
-      } else if constexpr (D == 2 && P == 2 && TX * TY == 32 && PH <= 1) {
-        // 16-byte pairs when every state pointer allows them
-        auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-        const bool vec = al(Uin) && (mode == 0 ? al(f_out) : al(Un) && al(Uacc) && al(Uout));
-        if (vec) {
-          kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 0, true> : k_stage<D, P, PH, FL, 1, TX, TY, 0, true>;
-          if (s.precision == 1)
-            kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 1, true> : k_stage<D, P, PH, FL, 1, TX, TY, 1, true>;
-          if (s.precision == 2)
-            kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 2, true> : k_stage<D, P, PH, FL, 1, TX, TY, 2, true>;
-        } else {
-          if (s.precision == 1)
-            kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 1> : k_stage<D, P, PH, FL, 1, TX, TY, 1>;
-          if (s.precision == 2)
-            kern = mode == 0 ? k_stage<D, P, PH, FL, 0, TX, TY, 2> : k_stage<D, P, PH, FL, 1, TX, TY, 2>;
-        }
-      }
-      // persistent grid: as many blocks as fit on the device at once
-      int nb = ntiles;
-      if (DGX_STAGE_PERSIST) {
-        int per_cu = 0, dev = 0, cus = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0) == hipSuccess && per_cu > 0)
-          nb = std::min(ntiles, per_cu * cus);
-      }
-      a.xcd_bands = (ntiles % 8 == 0 && nb % 8 == 0) ? 1 : 0;
-      // the epilogue's cell means: RK stages of 2D p=2 two-fluid tiles on the
-      // matrix-core element phases with the shared Minv (k_stage's MFW path)
-      constexpr bool mfw = D == 2 && P == 2 && PH == 1 && (TX * TY) % 16 == 0;
-      a.means = nullptr;
-      a.uavg = nullptr;
-      if (mfw && mode == 1 && means && s.t.mlp_vinv && s.t.minv_stride == 0 &&
-          (s.precision >= 1 || DGX_STAGE_MFMA64)) {
-        a.means = means;
-        a.uavg = uavg;
-        a.psens = psens;
-        if (means_done) *means_done = true;
-      }
-      hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, st, a);
+    constexpr int P = decltype(p)::value, FL = decltype(fl)::value;
+    const dim3 grid(8 * ((ntiles + 7) / 8)), block(256);  // whole bands (tile_of)
+    auto run = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, block, 0, st, a);
       return hipGetLastError();
     };
-    if constexpr (D == 1) {
-      if (c.tx == TileShape<1>::TX_SMALL) return go(std::integral_constant<int, TileShape<1>::TX_SMALL>{});
+    if constexpr (D == 2 && P >= 2) {
+      // 16-byte pairs when every state pointer and row allows them: rows start
+      // (and, ragged, end) on pairs when an element is a whole number of them
+      // or the grid has an even number of columns
+      constexpr bool even = Vol<D, P, PH>::NU % 2 == 0;
+      auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+      const bool vec = (even || c.nx % 2 == 0) && al(Uin) &&
+                       (mode == 0 ? al(f_out) : al(Un) && al(Uacc) && al(Uout));
+      if constexpr (P == 2 && PH == 1) {
+        // the epilogue's cell means: RK stages with the shared Minv
+        if (mode == 1 && means && s.t.mlp_vinv && s.t.minv_stride == 0) {
+          a.means = means;
+          a.uavg = uavg;
+          a.psens = psens;
+          if (means_done) *means_done = true;
+        }
+      }
+      if constexpr (P == 2 && PH <= 1) {
+        if (s.precision == 1)
+          return mode == 0 ? (vec ? run(k_stage_mfma<P, PH, FL, 0, 1, true, false>) : run(k_stage_mfma<P, PH, FL, 0, 1, false, false>))
+                           : (vec ? run(k_stage_mfma<P, PH, FL, 1, 1, true, false>) : run(k_stage_mfma<P, PH, FL, 1, 1, false, false>));
+        if (s.precision == 2)
+          return mode == 0 ? (vec ? run(k_stage_mfma<P, PH, FL, 0, 2, true, false>) : run(k_stage_mfma<P, PH, FL, 0, 2, false, false>))
+                           : (vec ? run(k_stage_mfma<P, PH, FL, 1, 2, true, false>) : run(k_stage_mfma<P, PH, FL, 1, 2, false, false>));
+      }
+      // states that cannot be paired (rare) take the ragged instance on whole tiles too
+      if (!vec) return mode == 0 ? run(k_stage_mfma<P, PH, FL, 0, 0, false, true>) : run(k_stage_mfma<P, PH, FL, 1, 0, false, true>);
+      if (ragged) return mode == 0 ? run(k_stage_mfma<P, PH, FL, 0, 0, true, true>) : run(k_stage_mfma<P, PH, FL, 1, 0, true, true>);
+      return mode == 0 ? run(k_stage_mfma<P, PH, FL, 0, 0, true, false>) : run(k_stage_mfma<P, PH, FL, 1, 0, true, false>);
+    } else {
+      auto go = [&](auto txc) -> hipError_t {
+        constexpr int TX = decltype(txc)::value, TY = TileShape<D>::TY;
+        if constexpr (D == 2) {
+          if (ragged)
+            return mode == 0 ? run(k_stage<D, P, PH, FL, 0, TX, TY, true>) : run(k_stage<D, P, PH, FL, 1, TX, TY, true>);
+        } else {
+          if (ragged) return hipErrorInvalidValue;  // 1D: the whole-step or the face + element kernels
+        }
+        return mode == 0 ? run(k_stage<D, P, PH, FL, 0, TX, TY, false>) : run(k_stage<D, P, PH, FL, 1, TX, TY, false>);
+      };
+      if constexpr (D == 1) {
+        if (c.tx == TileShape<1>::TX_SMALL) return go(std::integral_constant<int, TileShape<1>::TX_SMALL>{});
+      }
+      return go(std::integral_constant<int, TileShape<D>::TX>{});
     }
-    return go(std::integral_constant<int, TileShape<D>::TX>{});
   });
 }
-
-
 #define DGX_STAGE_PHYS(PH)                                                                                        \
   template hipError_t launch_stage_phys<PH>(const Solver&, int, int, const double*, const double*, double*, double*, \
                                             const double*, double*, hipStream_t, double*, double*, double*, bool*);

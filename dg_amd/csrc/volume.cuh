@@ -301,44 +301,121 @@ __device__ inline f32x4_t mma_bf16x3(const bf16x4_t& ah, const bf16x4_t& al, con
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, bh, c, 0, 0, 0);
 }
 
-// Doubles of per-wave LDS that vol_mfma_wave needs: the alpha source of four
-// elements (multifluid, FP64), then 16 flux rows of one direction in T
-// (16 points, padded).
-template <typename T, int PH>
-constexpr int vol_wave_lds() { return (PH ? 4 * 16 : 0) + (16 * 17 * (int)sizeof(T) + 7) / 8; }
+// Shape of the matrix-core element phases of 2D order P with physics PH.
+template <int P, int PH>
+struct VolMfma {
+  using V = Vol<2, P, PH>;
+  static constexpr int NF = V::NF, Ns = V::Ns, NG = V::NG, NNC = V::NNC;
+  static constexpr int NX = NF - 4;             // fields after rho, momenta and E
+  static constexpr int NXC = NX - NNC;          // of them, in conservation form (the first)
+  static constexpr int CB = (NG + 15) / 16;     // blocks of 16 Gauss points (columns of the map)
+  static constexpr int KN = (Ns + 3) / 4;       // steps over nodes
+  static constexpr int KG = (NG + 3) / 4;       // steps over Gauss points
+  static constexpr int KP = 4 * KG + 1;         // row of flux values, padded
+  static constexpr int NSR = NNC + 2 * NXC;     // row sets staged for the fields after E
+};
 
+// Doubles of per-wave LDS that vol_mfma_wave needs: 16 flux rows of one
+// direction in T, and, apart, 8 rows for each row set of the fields after E.
+template <typename T, int P>
+constexpr int vol_wave_flux() { return (16 * VolMfma<P, 0>::KP * (int)sizeof(T) + 7) / 8; }
+template <int P, int PH>
+constexpr int vol_wave_extra() { return VolMfma<P, PH>::NSR * 8 * VolMfma<P, PH>::KP; }
 
-// Element phases of a tile of NT 2D p=2 elements (256 threads, NT a multiple
-// of 16) on the matrix cores, contractions in T: double for the FP64 path,
-// float for the mixed-precision mode (FP32 inputs and accumulation; the
-// pointwise flux, the alpha terms, the face sums and everything after stay
-// FP64).
+// The lane's operands of the element phases, from the tables in global
+// memory: column (or B-side) index c = l % 16, contraction index 4s + l / 16.
+// Loaded before the block barrier that the phases wait at.
+template <typename T, int P, int PH, typename TM = T>
+struct VolOps {
+  using M = VolMfma<P, PH>;
+  TM phi[M::CB][M::KN];
+  T dw[2][M::KG];
+  double minv[M::KN];
+  double xphi[M::NX ? M::CB : 1][M::KN], dphi[M::NNC ? 2 : 1][M::NNC ? M::CB : 1][M::KN], pw[M::NNC ? M::KG : 1];
+  __device__ inline void load(const double* __restrict__ phi_g, const double* __restrict__ dphi_g,
+                              const double* __restrict__ phi_w, const double* __restrict__ dphi_w,
+                              const double* __restrict__ Minv, int tid) {
+    constexpr int Ns = M::Ns, NG = M::NG;
+    const int l = tid & 63, c = l & 15, q = l >> 4;
+    // entries outside a table are 0, read from its first entry: no branch
+    auto at = [](const double* __restrict__ t, bool in, int i) {
+      const double v = t[in ? i : 0];
+      return in ? v : 0.0;
+    };
+#pragma unroll
+    for (int s = 0; s < M::KN; ++s) {
+      const int k = 4 * s + q;
+#pragma unroll
+      for (int b = 0; b < M::CB; ++b) {
+        const int g = 16 * b + c;
+        const bool in = (Ns % 4 == 0 || k < Ns) && (NG % 16 == 0 || g < NG);
+        const double v = at(phi_g, in, g + k * NG);
+        phi[b][s] = (TM)v;
+        if constexpr (M::NX > 0) xphi[b][s] = v;
+        if constexpr (M::NNC > 0)
+#pragma unroll
+          for (int al = 0; al < 2; ++al) dphi[al][b][s] = at(dphi_g, in, (g * 2 + al) + k * NG * 2);
+      }
+      minv[s] = Minv ? at(Minv, k < Ns && c < Ns, k * Ns + c) : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < M::KG; ++s) {
+      const int g = 4 * s + q;
+      const bool in = (NG % 4 == 0 || g < NG) && (Ns == 16 || c < Ns);
+#pragma unroll
+      for (int al = 0; al < 2; ++al) dw[al][s] = (T)at(dphi_w, in, c * NG * 2 + g * 2 + al);
+      if constexpr (M::NNC > 0) pw[s] = at(phi_w, in, g + c * NG);
+    }
+  }
+};
+
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Element phases of a tile of 32 2D elements of order P = 2 or 3 (256
+// threads) on the matrix cores, contractions of rho, momenta and E in T:
+// double for the FP64 path, float for the mixed-precision mode (FP32 inputs
+// and accumulation; the pointwise flux, the fields after E, the face sums and
+// everything after stay FP64).
 //   map        Ug[(el,f)][g]  = sum_i U[el][f][i] phi[g][i]         fields 0..3
-//   flux       fe[(el,f)][g,al] = J_e sum_k invJac[al][k] f_k(Ug)    in registers
+//   flux       fe[(el,f)][g,al] = sum_k (J_e invJac)[al][k] f_k(Ug)  in registers
+//              (sGeo holds J_e invJac per element)
 //   integrate  R[(el,f)][i]   = sum_{al} sum_g fe[(el,f)][g,al] dphi_w[g,al][i]
-// Wave w owns elements 4w..4w+3 of every group of 16.  After the map each
-// lane holds the four conserved fields of one element at one Gauss point, so
-// the flux needs no exchange; the scaled fluxes pass through the wave's own
-// LDS rows, one direction at a time, into the integration, whose result
-// registers plus the face sums are the right-hand side, written to sU.
-// The integration operand (dphi_w, [i*NG*D + g*D + al]) is read from global
-// memory into registers once.  Multifluid adds alpha and its reference
-// gradient at the point (FP64 sums over the 9 nodes) and the alpha source
-// integrated against phi_w (FP64).  With minv (the shared mass-matrix
-// inverse in LDS, [ii*Ns + i]) and dte (Dt per element), the right-hand side
-// is then replaced by du = dte * Minv * R, again on the FP64 matrix cores
-// (A = R rows read back from sU, B = Minv; alpha by FP64 sums).  No block
-// barrier: every exchange stays inside the wave.  sWork needs
-// 4 * vol_wave_lds<T, PH>() doubles.
-// SPLIT (T = TM = float): the map and the integration as split-BF16
+// Wave w owns elements 4w..4w+3 of both groups of 16.  After the map each
+// lane holds the four conserved fields of one element at one Gauss point (two
+// at p = 3: 25 points in two column blocks), so the flux needs no exchange;
+// the scaled fluxes pass through the wave's own LDS rows, one direction at a
+// time, into the integration, whose result registers plus the face sums are
+// the right-hand side, written to sU.
+//
+// The fields after E (alpha; rho phic and phinc; alpha and beta) of the
+// wave's eight elements are rows of matrix products of their own, both groups
+// at once: row el8 + 8x (el8 = 4*group + element, x the field) puts field x of
+// element l/16 of group g into result register 2x + g of lane l.  Their
+// values and reference gradients at the points, the sources against phi_w,
+// the flux of a conservative one against dphi_w and their share of Dt*Minv
+// are 9 + 4 + 3 products of a wave at p = 2 two-fluid; as sums on the vector
+// units they took 104 FMAs and 146 LDS reads of a lane (a third of the
+// phase's), and their tables 4.6 KB of LDS.
+//
+// With with_minv the right-hand side is then replaced by du = dte * Minv * R,
+// again on the FP64 matrix cores (A = R rows read back from sU).  No block
+// barrier: every exchange stays inside the wave.  face(el, q) gives the
+// face sums q[0..NF) of the lane's node (c) of tile element el.  sFlux needs
+// 4 * vol_wave_flux<T, P>() doubles, sExtra 4 * vol_wave_extra<P, PH>().
+// SPLIT (T = TM = float, P = 2): the map and the integration as split-BF16
 // products on v_mfma_f32_16x16x16_bf16 (K = 16 per instruction: A lane l =
 // row l%16, k = 4(l/16)+0..3; B lane l = column l%16, same k; D as the FP32
 // 16x16x4 layout), three instructions per contraction block.
-template <typename T, int PH, int NT, int SU, int SQ, int NGEO, typename TM = T, bool SPLIT = false>
-__device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __restrict__ dphi_w, double* sU,
-                              const double* sGeo, const double* sQ, double* sWork, const int* sNodeQ, int tid,
-                              const double* minv = nullptr, const double* dte = nullptr) {
-  static_assert(!SPLIT || (std::is_same<T, float>::value && std::is_same<TM, float>::value),
+template <typename T, int P, int PH, int SU, typename TM, bool SPLIT, typename Face>
+__device__ __forceinline__ void vol_mfma_wave(const VolOps<T, P, PH, TM>& op, const double* __restrict__ phi_g,
+                                              const double* __restrict__ dphi_w, double* sU, const double* sGeo,
+                                              double* sFlux, double* sExtra, int tid, bool with_minv,
+                                              const double* dte, Face&& face) {
+  static_assert(!SPLIT || (P == 2 && std::is_same<T, float>::value && std::is_same<TM, float>::value),
                 "split-BF16 accumulates in FP32");
   // TM: type of the map (T unless set), T: type of the integration.  On gfx950
   // the FP32 16x16x4 integration measured slower than the FP64 one (volume
@@ -346,25 +423,14 @@ __device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __rest
   // as fast as the FP64 map.
   using M = Mfma16<T>;
   using MM = Mfma16<TM>;
-  constexpr int NF = 4 + PH, Ns = 9, NG = 16, D = 2, KP = NG + 1, Ms = 3;
-  static_assert(NT % 16 == 0, "groups of 16 elements, four per wave");
-  static_assert(PH <= 1, "single-fluid and two-fluid states only");
+  using M64 = Mfma16<double>;
+  using S = VolMfma<P, PH>;
+  constexpr int NF = S::NF, Ns = S::Ns, NG = S::NG, D = 2, KP = S::KP, NX = S::NX, NXC = S::NXC, NNC = S::NNC;
+  constexpr int CB = S::CB, KN = S::KN, KG = S::KG;
   const int w = tid >> 6, l = tid & 63, c = l & 15, q = l >> 4;
-  double* S = sWork + w * vol_wave_lds<T, PH>();
-  T* F = reinterpret_cast<T*>(S + (PH ? 4 * NG : 0));
-  TM bphi[3];
-  T bdw[8];
-#pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    const int k = 4 * s + q;
-    bphi[s] = k < Ns ? (TM)t.phi[c + k * NG] : TM(0);
-  }
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {  // direction s/4, points 4(s%4)+q
-    const int g = 4 * (s & 3) + q, al = s >> 2;
-    bdw[s] = c < Ns ? (T)dphi_w[c * NG * D + g * D + al] : T(0);
-  }
-  const int a_el = MM::el(c), a_f = MM::field(c);
+  T* F = reinterpret_cast<T*>(sFlux + w * vol_wave_flux<T, P>());
+  double* X = sExtra + w * vol_wave_extra<P, PH>();
+  auto elem = [&](int e8) { return 16 * (e8 >> 2) + 4 * w + (e8 & 3); };  // tile element of this wave's e8-th
   // split-BF16 B operands: phi[g = c][i = 4q+j] for the map, dphi_w[i = c][g = 4q+j][al] for the integration
   bf16x4_t sphi_h = {0, 0, 0, 0}, sphi_l = {0, 0, 0, 0}, sdw_h[2], sdw_l[2];
   if constexpr (SPLIT) {
@@ -372,7 +438,7 @@ __device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __rest
     for (int j = 0; j < 4; ++j) {
       const int k = 4 * q + j;
       short h, lo;
-      bf16_split(k < Ns ? (float)t.phi[c + k * NG] : 0.0f, h, lo);
+      bf16_split(k < Ns ? (float)phi_g[c + k * NG] : 0.0f, h, lo);
       sphi_h[j] = h;
       sphi_l[j] = lo;
 #pragma unroll
@@ -383,18 +449,36 @@ __device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __rest
       }
     }
   }
-  // Minv operand: column c (output node), rows k = 4s + q (input node)
-  double bminv[3];
+  // ---- the fields after E at the points, both groups: row c of A
+  M64::V4 xv[NX ? CB : 1], xd[NNC ? 2 : 1][NNC ? CB : 1];
+  const int xe = elem(c & 7), xf = 4 + (c >> 3);  // this lane's row: element and field (rows of absent fields are 0)
+  if constexpr (NX > 0) {
 #pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    const int k = 4 * s + q;
-    bminv[s] = (minv && k < Ns && c < Ns) ? minv[k * Ns + c] : 0.0;
+    for (int b = 0; b < CB; ++b) {
+      xv[b] = {0.0, 0.0, 0.0, 0.0};
+      if constexpr (NNC > 0) xd[0][b] = xd[1][b] = {0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll
+    for (int s = 0; s < KN; ++s) {
+      const int k = 4 * s + q;
+      const double a = (Ns % 4 == 0 || k < Ns) && (NX == 2 || c < 8) ? sU[xe * SU + xf * Ns + k] : 0.0;
+#pragma unroll
+      for (int b = 0; b < CB; ++b) {
+        xv[b] = M64::mma(a, op.xphi[b][s], xv[b]);
+        if constexpr (NNC > 0)
+#pragma unroll
+          for (int al = 0; al < D; ++al) xd[al][b] = M64::mma(a, op.dphi[al][b][s], xd[al][b]);
+      }
+    }
   }
-#pragma unroll 1
-  for (int b = 0; b < NT; b += 16) {
-    const int e_base = b + 4 * w, el = e_base + q;
+  const int a_el = MM::el(c), a_f = MM::field(c);
+#pragma unroll
+  for (int grp = 0; grp < 2; ++grp) {
+    const int e_base = 16 * grp + 4 * w, el = e_base + q;
     // ---- map
-    typename MM::V4 acc = {TM(0), TM(0), TM(0), TM(0)};
+    typename MM::V4 acc[CB];
+#pragma unroll
+    for (int b = 0; b < CB; ++b) acc[b] = {TM(0), TM(0), TM(0), TM(0)};
     if constexpr (SPLIT) {
       bf16x4_t ah, alo;
 #pragma unroll
@@ -405,59 +489,66 @@ __device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __rest
         ah[j] = h;
         alo[j] = lo;
       }
-      acc = mma_bf16x3(ah, alo, sphi_h, sphi_l, acc);
+      acc[0] = mma_bf16x3(ah, alo, sphi_h, sphi_l, acc[0]);
     } else {
 #pragma unroll
-      for (int s = 0; s < 3; ++s) {
+      for (int s = 0; s < KN; ++s) {
         const int k = 4 * s + q;
-        const TM a = k < Ns ? (TM)sU[(e_base + a_el) * SU + a_f * Ns + k] : TM(0);
-        acc = MM::mma(a, bphi[s], acc);
+        const TM a = (Ns % 4 == 0 || k < Ns) ? (TM)sU[(e_base + a_el) * SU + a_f * Ns + k] : TM(0);
+#pragma unroll
+        for (int b = 0; b < CB; ++b) acc[b] = MM::mma(a, op.phi[b][s], acc[b]);
       }
     }
-    double ug[NF], dua[D] = {0.0, 0.0};
-#pragma unroll
-    for (int v = 0; v < 4; ++v) ug[v] = (double)acc[v];
-    if constexpr (PH == 1) {
-      const double* ua = sU + el * SU + 4 * Ns;
-      double al = 0, d0 = 0, d1 = 0;
-#pragma unroll
-      for (int k = 0; k < Ns; ++k) {
-        const double uk = ua[k];
-        al += t.phi[c + k * NG] * uk;
-        d0 += t.dphi[(c * D + 0) + k * NG * D] * uk;
-        d1 += t.dphi[(c * D + 1) + k * NG * D] * uk;
-      }
-      ug[4] = al;
-      dua[0] = d0;
-      dua[1] = d1;
-    }
-    // ---- flux of element el at point g = c with metric terms
-    T fe[4][D];
+    // ---- flux of element el at point g = 16b + c with metric terms
+    T fe[CB][4][D];
     {
-      const double Je = sGeo[el * NGEO];
-      const double* ij = sGeo + el * NGEO + 1;
-      double fx[NF * D], salpha;
-      volume_flux<2, PH>(ug, dua, ij, fx, &salpha);
+      const double ij[4] = {sGeo[el * 4], sGeo[el * 4 + 1], sGeo[el * 4 + 2], sGeo[el * 4 + 3]};  // J_e invJac
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+      for (int b = 0; b < CB; ++b) {
+        double ug[NF], dua[(NNC ? NNC : 1) * D], fx[NF * D], snc[NNC ? NNC : 1];
 #pragma unroll
-        for (int al = 0; al < D; ++al) {
-          double sol = 0.0;
+        for (int v = 0; v < 4; ++v) ug[v] = (double)acc[b][v];
+        // points past the last (p = 3) repeat element q's first-block point
+        const bool in = NG % 16 == 0 || 16 * b + c < NG;
+        if constexpr (NG % 16 != 0) {
+          if (b == CB - 1)
 #pragma unroll
-          for (int k = 0; k < D; ++k) sol += ij[al * D + k] * fx[f * D + k] * Je;
-          fe[f][al] = (T)sol;
+            for (int v = 0; v < 4; ++v) ug[v] = in ? ug[v] : (double)acc[0][v];
         }
-      if constexpr (PH == 1) S[q * NG + c] = salpha * Je;
+#pragma unroll
+        for (int x = 0; x < NX; ++x) ug[4 + x] = in ? xv[b][2 * x + grp] : xv[0][2 * x + grp];
+#pragma unroll
+        for (int m = 0; m < NNC; ++m)
+#pragma unroll
+          for (int al = 0; al < D; ++al) dua[m * D + al] = xd[al][b][2 * (NXC + m) + grp];
+        volume_flux<2, PH>(ug, dua, ij, fx, snc);
+        const bool row = NG % 16 == 0 || 16 * b + c < 4 * KG;  // within the padded row
+#pragma unroll
+        for (int f = 0; f < 4 + NXC; ++f)
+#pragma unroll
+          for (int al = 0; al < D; ++al) {
+            double sol = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) sol += ij[al * D + k] * fx[f * D + k];
+            if (!in) sol = 0.0;
+            if (f < 4) fe[b][f < 4 ? f : 0][al] = (T)sol;
+            else if (row) X[((NNC + al) * 8 + 4 * grp + q) * KP + 16 * b + c] = sol;
+          }
+#pragma unroll
+        for (int m = 0; m < NNC; ++m)
+          if (row) X[(m * 8 + 4 * grp + q) * KP + 16 * b + c] = in ? snc[m] : 0.0;
+      }
     }
     // ---- integration, one direction at a time through this wave's rows
     typename M::V4 r = {T(0), T(0), T(0), T(0)};
 #pragma unroll
     for (int al = 0; al < D; ++al) {
 #pragma unroll
-      for (int f = 0; f < 4; ++f) F[M::row(q, f) * KP + c] = fe[f][al];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int b = 0; b < CB; ++b)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+          if (NG % 16 == 0 || 16 * b + c < 4 * KG) F[M::row(q, f) * KP + 16 * b + c] = fe[b][f][al];
+      wave_sync();
       if constexpr (SPLIT) {
         bf16x4_t ah, alo;
 #pragma unroll
@@ -470,64 +561,171 @@ __device__ void vol_mfma_wave(const VolTables<2, 2, PH>& t, const double* __rest
         r = mma_bf16x3(ah, alo, sdw_h[al], sdw_l[al], r);
       } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) r = M::mma(F[c * KP + 4 * s + q], bdw[4 * al + s], r);
+        for (int s = 0; s < KG; ++s) r = M::mma(F[c * KP + 4 * s + q], op.dw[al][s], r);
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();  // the rows are rewritten next
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      wave_sync();  // the rows are rewritten next
     }
-    double sa = 0;
-    if constexpr (PH == 1) {
-      if (c < Ns) {
+    if (Ns == 16 || c < Ns) {
+      double qs[NF];
+      face(el, qs);
 #pragma unroll
-        for (int g = 0; g < NG; ++g) sa += S[q * NG + g] * t.pw[g * Ns + c];
-      }
+      for (int v = 0; v < 4; ++v) sU[el * SU + v * Ns + c] = (double)r[v] + qs[v];
+#pragma unroll
+      for (int x = 0; x < NX; ++x) sU[el * SU + (4 + x) * Ns + c] = qs[4 + x];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // F and S are rewritten by the next group
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (c < Ns) {
-      const int q0 = sNodeQ[2 * c], q1 = sNodeQ[2 * c + 1];
-      auto face = [&](int f) {
-        double qs = 0.0;
-        if (q0 >= 0) qs += sQ[el * SQ + q0 + f * Ms];
-        if (q1 >= 0) qs += sQ[el * SQ + q1 + f * Ms];
-        return qs;
-      };
+  }
+  // ---- the fields after E: sources and fluxes integrated, both groups
+  if constexpr (NX > 0) {
+    M64::V4 rx = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int v = 0; v < 4; ++v) sU[el * SU + v * Ns + c] = (double)r[v] + face(v);
-      if constexpr (PH == 1) sU[el * SU + 4 * Ns + c] = sa + face(4);
+    for (int s = 0; s < KG; ++s) {
+      const int g = 4 * s + q, x = c >> 3;
+      // rows of field x: its source (the last NNC), or nothing here
+      const int m = x - NXC;
+      const double a = (m >= 0 && m < NNC) ? X[(m * 8 + (c & 7)) * KP + g] : 0.0;
+      rx = M64::mma(a, op.pw[s], rx);
     }
-    if (minv) {
-      // du = dte * Minv R: rows (el, f) = el + 4f of the four elements, columns = nodes
-      using M64 = Mfma16<double>;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();  // the right-hand side of the four elements is in sU
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      M64::V4 du = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (NXC > 0) {
 #pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        const int k = 4 * s + q;
-        const double a = k < Ns ? sU[(e_base + M64::el(c)) * SU + M64::field(c) * Ns + k] : 0.0;
-        du = M64::mma(a, bminv[s], du);
-      }
-      double dua5 = 0.0;
-      if constexpr (PH == 1) {
-        if (c < Ns) {
+      for (int al = 0; al < D; ++al)
 #pragma unroll
-          for (int k = 0; k < Ns; ++k) dua5 += minv[k * Ns + c] * sU[el * SU + 4 * Ns + k];
+        for (int s = 0; s < KG; ++s) {
+          const double a = c < 8 ? X[((NNC + al) * 8 + c) * KP + 4 * s + q] : 0.0;
+          rx = M64::mma(a, (double)op.dw[al][s], rx);
         }
+    }
+    if (Ns == 16 || c < Ns)
+#pragma unroll
+      for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int grp = 0; grp < 2; ++grp) {
+          double* u = sU + (16 * grp + 4 * w + q) * SU + (4 + x) * Ns + c;
+          *u = rx[2 * x + grp] + *u;
+        }
+  }
+  if (with_minv) {
+    // du = dte * Minv R: rows (el, f) = el + 4f of the four elements, columns = nodes
+    wave_sync();  // the right-hand side of the eight elements is in sU
+    M64::V4 du[2], dx = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp) {
+      du[grp] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < KN; ++s) {
+        const int k = 4 * s + q;
+        const double a = (Ns % 4 == 0 || k < Ns)
+                             ? sU[(16 * grp + 4 * w + M64::el(c)) * SU + M64::field(c) * Ns + k]
+                             : 0.0;
+        du[grp] = M64::mma(a, op.minv[s], du[grp]);
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();  // every lane has read the right-hand side
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (c < Ns) {
+    }
+    if constexpr (NX > 0) {
+#pragma unroll
+      for (int s = 0; s < KN; ++s) {
+        const int k = 4 * s + q;
+        const double a = (Ns % 4 == 0 || k < Ns) && (NX == 2 || c < 8) ? sU[xe * SU + xf * Ns + k] : 0.0;
+        dx = M64::mma(a, op.minv[s], dx);
+      }
+    }
+    wave_sync();  // every lane has read the right-hand side
+    if (Ns == 16 || c < Ns)
+#pragma unroll
+      for (int grp = 0; grp < 2; ++grp) {
+        const int el = 16 * grp + 4 * w + q;
         const double d = dte[el];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sU[el * SU + v * Ns + c] = d * du[v];
-        if constexpr (PH == 1) sU[el * SU + 4 * Ns + c] = d * dua5;
+        for (int v = 0; v < 4; ++v) sU[el * SU + v * Ns + c] = d * du[grp][v];
+#pragma unroll
+        for (int x = 0; x < NX; ++x) sU[el * SU + (4 + x) * Ns + c] = d * dx[2 * x + grp];
+      }
+  }
+}
+
+// Node of the 2D p = 2 element (Gmsh order) at the lane's place of
+// vol_tensor_wave (column a = l % 4, row b = l / 16 of the lattice), or -1.
+__device__ inline int tensor_node(int l) {
+  const int a = l & 3, b = (l >> 4) & 3;
+  // rows of the lattice: 0 4 1 / 7 8 5 / 3 6 2
+  constexpr unsigned long long kNodes = 0xfff'f'f263'f587'f140ull;
+  const int n = (int)((kNodes >> (16 * b + 4 * a)) & 15);
+  return n == 15 ? -1 : n;
+}
+
+// The same phases for P = 2 in FP64 as chains of 4x4 products: three nodes and
+// four Gauss points per direction fit v_mfma_f64_4x4x4_4b_f64, four
+// independent 4x4x4 products, one element each.  Its operands (lane l = 16r +
+// 4e + c: A row c, B column c, contraction index r, D row r, column c, of
+// block e) make a result usable as the next product's A with its row index
+// contracted, so a field goes through both directions, to the points and
+// back, without leaving its registers:
+//   u[b][a] -> A1[a][gy] = sum_b u[b][a] V[gy][b] -> A2[gy][gx] = sum_a A1[a][gy] V[gx][a]
+// (derivative tables in place of V for the gradients), the flux in the lane of
+// its point, the test integrals and the mass matrix the same way.  Lane:
+// element e of the wave's group, node (a = c, b = r) or point (gx = c, gy = r).
+//
+// FP64 matrix and vector instructions share the FP64 units on this chip
+// (measured: 64 cycles a 16x16x4 product whatever runs beside it, while the
+// vector FMAs beside it drop from one in 2.8 cycles to one in 9.9; 19 cycles a
+// 4x4x4), so what counts is their sum: 82 products of 16 cycles a wave against
+// 44 of 64 for two-fluid with 16x16 tiles, whose rows and columns padding half
+// fills; and no flux rows (8.7 KB), no tables (7.6 KB) and no barriers in LDS.
+// tab: the tables in LDS, [table][r*4 + c]: V, V', V*w, V'*w, inverse 1D mass
+// matrix (tensor_tables).  dtj: Dt / J per element.
+constexpr int kTensorTables = 5;
+template <int PH, int SU, typename Face>
+__device__ __forceinline__ void vol_tensor_wave(const double* tab, double* sU, const double* sGeo, int tid,
+                                                bool with_minv, const double* dtj, Face&& face) {
+  using V = Vol<2, 2, PH>;
+  constexpr int NF = V::NF, Ns = V::Ns, NFX = V::NFX, NNC = V::NNC, D = 2;
+  const int w = tid >> 6, l = tid & 63, r = l >> 4, e = (l >> 2) & 3, c = l & 3;
+  auto mma = [](double a, double b, double acc) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, acc, 0, 0, 0); };
+  const double bV = tab[r * 4 + c], bD = tab[16 + r * 4 + c], bVw = tab[32 + r * 4 + c], bDw = tab[48 + r * 4 + c],
+               bM = tab[64 + r * 4 + c];
+  const int node = tensor_node(l);
+  const bool on = node >= 0;
+#pragma unroll
+  for (int grp = 0; grp < 2; ++grp) {
+    const int el = 16 * grp + 4 * w + e;
+    double* ue = sU + el * SU + (on ? node : 0);
+    double u[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const double v = ue[f * Ns];
+      u[f] = on ? v : 0.0;
+    }
+    double ug[NF], dua[(NNC ? NNC : 1) * D];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const double a1 = mma(u[f], bV, 0.0);
+      ug[f] = mma(a1, bV, 0.0);
+      if (f >= NFX) {
+        dua[(f - NFX) * D] = mma(a1, bD, 0.0);
+        dua[(f - NFX) * D + 1] = mma(mma(u[f], bD, 0.0), bV, 0.0);
       }
     }
+    const double ij[4] = {sGeo[el * 4], sGeo[el * 4 + 1], sGeo[el * 4 + 2], sGeo[el * 4 + 3]};  // J_e invJac
+    double fx[NF * D], snc[NNC ? NNC : 1], R[NF];
+    volume_flux<2, PH>(ug, dua, ij, fx, snc);
+#pragma unroll
+    for (int f = 0; f < NFX; ++f) {
+      const double f0 = ij[0] * fx[f * D] + ij[1] * fx[f * D + 1], f1 = ij[2] * fx[f * D] + ij[3] * fx[f * D + 1];
+      R[f] = mma(mma(f0, bVw, 0.0), bDw, 0.0);
+      R[f] = mma(mma(f1, bDw, 0.0), bVw, R[f]);
+    }
+#pragma unroll
+    for (int m = 0; m < NNC; ++m) R[NFX + m] = mma(mma(snc[m], bVw, 0.0), bVw, 0.0);
+    double qs[NF];
+    face(el, qs);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) R[f] = on ? R[f] + qs[f] : 0.0;
+    if (with_minv) {
+      const double d = dtj[el];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) R[f] = d * mma(mma(R[f], bM, 0.0), bM, 0.0);
+    }
+    if (on)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) ue[f * Ns] = R[f];
   }
 }
 
