@@ -449,7 +449,7 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
   ok = ok && alloc(s, &s.Qe, (size_t)NE * NN * s.NF * s.M_s) && alloc(s, &s.Uacc, S) && alloc(s, &s.Ustar, S) &&
        alloc(s, &s.work, S) && alloc(s, &s.work2, S) && alloc(s, &s.Uavg, (size_t)NE * s.NF) &&
        alloc(s, &s.sensors, (size_t)NE) && alloc(s, &s.sens_tgt, (size_t)2 * NE) &&
-       alloc(s, &s.sens_act, (size_t)3 * NE) && alloc(s, &s.flag, 4) && alloc(s, &s.sens_changed, kRelaxBatch) && alloc(s, &s.flag_list, (size_t)NE) &&
+       alloc(s, &s.flag, 4) && alloc(s, &s.flag_list, (size_t)NE) &&
        alloc(s, &s.dscratch, 8) && alloc(s, &s.time_state, 8) &&
        alloc(s, &s.cons_partial, conservation_scratch_doubles()) &&
        alloc(s, &s.dt_partial, ((size_t)NE * Ns + 255) / 256 + 1) &&
@@ -666,10 +666,13 @@ static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, 
   // means, and the indicator that follows skips its own pass over the state
   double* means = (limiter == 8 && s.mlp && s.fuse_means) ? s.mlp_avg : nullptr;
   bool means_ready = false;
+  // the same for the averages of the limiters that start with the sensor
+  const bool senses = limiter == 3 || limiter == 4 || limiter == 6 || limiter == 7;
+  double* uavg = senses || (means && s.shock_guard_on()) ? s.Uavg : nullptr;
   auto limit = [&](double* V) {
-    s.means_of = means_ready ? V : nullptr;
+    (senses ? s.avgs_of : s.means_of) = means_ready ? V : nullptr;
     const dgx_status q = timed_limit(s, limiter, V, st);
-    s.means_of = nullptr;
+    s.means_of = s.avgs_of = nullptr;
     return q;
   };
   double* cur = U;
@@ -680,8 +683,8 @@ static dgx_status rk4_step(Solver& s, double* U, const double* dt, int limiter, 
     cur = Uout;
     if (tiled) {
       KernelTimer kt(s, 4, st);
-      if (!hip_ok(launch_stage(s, 1, k, Uin, U, s.Uacc, Uout, dt, nullptr, st, means,
-                               means && s.shock_guard_on() ? s.Uavg : nullptr, s.mlp_psens, &means_ready),
+      if (!hip_ok(launch_stage(s, 1, k, Uin, U, s.Uacc, Uout, dt, nullptr, st, means, uavg,
+                               s.mlp_psens, &means_ready),
                   "tile kernel"))
         return DGX_EDEVICE;
       continue;

@@ -37,14 +37,14 @@ hipError_t compat_m2i(int D, int N_s1D, int N_E, int N_N, const int* nb, int off
 
 static dgx_config g_cfg = {1, 2, DGX_MULTIFLUID, DGX_RUSANOV};
 
-// Fixed device scratch of dgx_calc_sensors_noalloc: five ints per element
-// (hit targets, hit values, two activity vectors, initial flags) for up to
-// kSensorsNoallocMaxElements elements, then the sweep flag.  Each GPU the
-// library runs on holds its own copy (40 MiB) until the process ends.  Host
+// Fixed device scratch of dgx_calc_sensors_noalloc: three ints per
+// element (hit targets, hit values, initial flags) for up to
+// kSensorsNoallocMaxElements elements.  Each GPU the library runs on holds its
+// own copy (24 MiB) until the process ends.  Host
 // code never uses the array's name as an address: noalloc_scratch() looks up
 // each device's copy once, with that device current.
 constexpr long kSensorsNoallocMaxElements = 1L << 21;
-static __device__ __align__(256) int scratch[5 * kSensorsNoallocMaxElements + 64];
+static __device__ __align__(256) int scratch[3 * kSensorsNoallocMaxElements];
 
 static std::mutex g_scratch_mu;
 static int* g_scratch_dev[64];  // the array's address on each device, once looked up
@@ -404,20 +404,13 @@ void Lcalc_sensors(int N_E, int N_N, dgx_bool sensor1, double thresh1, dgx_bool 
   tmp.N_E = N_E;
   tmp.N_N = N_N;
   int* buf = nullptr;
-  int* flag = nullptr;
-  if (!hip_ok(hipMalloc(&buf, sizeof(int) * 5 * (size_t)N_E), "Lcalc_sensors") ||
-      !hip_ok(hipMalloc(&flag, sizeof(int)), "Lcalc_sensors")) {
-    hipFree(buf);
-    return;
-  }
-  tmp.flag = flag;
+  if (!hip_ok(hipMalloc(&buf, sizeof(int) * 3 * (size_t)N_E), "Lcalc_sensors")) return;
   int on[3] = {sensor1, sensor2, sensor3};
   double th[3] = {thresh1, thresh2, thresh3};
   hipError_t e = compat_sensors(tmp, neighbors, Uavg, sensors, on, th, buf);
   if (e != hipSuccess) hip_ok(e, "Lcalc_sensors");
   finish("Lcalc_sensors");
   hipFree(buf);
-  hipFree(flag);
 }
 
 dgx_status dgx_calc_sensors_noalloc(int N_E, int N_N, dgx_bool sensor1, double thresh1, dgx_bool sensor2,
@@ -440,9 +433,7 @@ dgx_status dgx_calc_sensors_noalloc(int N_E, int N_N, dgx_bool sensor1, double t
   tmp.D = g_cfg.dim;
   tmp.N_E = N_E;
   tmp.N_N = N_N;
-  // [0, 5*N_E): hit targets and values, two activity vectors, initial flags;
-  // the sweep flag after the largest such span, so its offset never moves
-  tmp.flag = base + 5 * (size_t)kSensorsNoallocMaxElements;
+  // [0, 3*N_E): hit targets and values, initial flags
   int on[3] = {sensor1, sensor2, sensor3};
   double th[3] = {thresh1, thresh2, thresh3};
   hipError_t e = compat_sensors(tmp, neighbors, Uavg, sensors, on, th, base);

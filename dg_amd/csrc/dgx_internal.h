@@ -70,10 +70,6 @@ struct Cart {
 
 enum KernelPath { PATH_AUTO = 0, PATH_GENERAL = 1, PATH_TILED = 2 };
 
-// Sensor relaxation sweeps queued per host read-back (the 1024x512
-// shock-bubble needs about three).
-constexpr int kRelaxBatch = 4;
-
 struct Solver {
   dgx_config cfg{};
   int D = 1, P = 1, NF = 3, N_s = 0, N_G = 0, M_s = 0, M_G = 0, N_N = 0, N_E = 0, M_T = 0, N1 = 0;
@@ -103,9 +99,7 @@ struct Solver {
   double* Uavg = nullptr;   // [e*NF+f]
   int* sensors = nullptr;   // [e]
   int* sens_tgt = nullptr;  // sensor resolution scratch [e*2]
-  int* sens_act = nullptr;  // [e*2] (ping-pong)
-  int* flag = nullptr;      // device flag / counters: [0] sensor relaxation, [2] flagged-element count
-  int* sens_changed = nullptr;  // [kRelaxBatch] change flags of a batch of sensor relaxation sweeps
+  int* flag = nullptr;      // device counters: [2] flagged-element count
   int* flag_list = nullptr; // [N_E] flagged elements (launch_limit_flagged)
   double* m2buf = nullptr;  // m2 limiting: 15 per-field arrays of N_E*N_s (allocated on first use)
   double* dscratch = nullptr;  // device scalars: [1] Dt, [2] the time of a device-timed CFL run; [4..7] {Dt, T} in two slots (1D)
@@ -128,6 +122,7 @@ struct Solver {
   // the state whose cell means mlp_avg holds, set by the RK driver between a
   // stage that emitted them and the indicator that reads them (else null)
   const double* means_of = nullptr;
+  const double* avgs_of = nullptr;  // likewise the state whose sensor averages Uavg holds, for launch_sensing
   bool fuse_means = true;      // RK stages emit the indicator's cell means (dgx_solver_set_fused_means)
   bool shock_guard = true;     // the indicator also flags the sensor's shock pairs (dgx_solver_set_shock_guard)
   double* mlp_psens = nullptr; // [e] the sensor's pressure from the cell averages (shock guard)
@@ -154,9 +149,10 @@ hipError_t launch_face_geometry(const Solver& s, hipStream_t st);
 // fused tile kernel (Cartesian meshes): same modes as launch_elem
 bool stage_tiles(int D, int nx, int ny, int* tx, int* ty);
 // means: also write the output tile's cell means of rho, p and alpha there
-// (2D p=2 two-fluid RK stages), and with uavg and psens the sensor's cell
-// averages and pressures;
-// *means_done tells whether the kernel did
+// (2D p=2 two-fluid RK stages), and with uavg the sensor's cell averages and
+// in psens their pressures.  uavg without means: only the averages (2D p=2,3
+// RK stages, not single fluid).  *means_done tells whether the kernel wrote
+// what was asked for
 hipError_t launch_stage(const Solver& s, int mode, int stage, const double* Uin, const double* Un, double* Uacc,
                         double* Uout, const double* dt_dev, double* f_out, hipStream_t st, double* means = nullptr,
                         double* uavg = nullptr, double* psens = nullptr, bool* means_done = nullptr);

@@ -13,13 +13,12 @@
 //   sensor_kernels.cu:19-163): the reference loops over elements in order and
 //   each element skips the test if an earlier element already flagged it,
 //   then overwrites its flagged neighbour.  The result depends on that order.
-//   Here it is reproduced deterministically in three phases:
+//   Here it is reproduced deterministically in two phases:
 //     k_sensor_hit    per element, the first neighbour test that fires
 //                     (independent of order);
-//     k_sensor_relax  "active" = not flagged by an earlier active element,
-//                     iterated to its fixed point (a DAG in element order);
 //     k_sensor_final  each element takes the value of its last writer in
-//                     element order.
+//                     element order, of those that no earlier element flagged
+//                     (sensor_runs).
 // Sensor-gated HR (Limiting::HRIlimiting, limiting.cc:596-634; hri1D,
 //   limiting_kernels.cu:322-427; copy_detected, sensor_kernels.cu:167-200).
 #pragma clang fp contract(off)
@@ -620,61 +619,88 @@ __global__ __launch_bounds__(256) void k_uavg(const double* __restrict__ U, long
 struct SensorTh {
   int on[3];
   double th[3];
+  double cut[3];  // sensor_cut of th
 };
 
 // First test that fires for element e (as if e is tested): tgt = neighbour
-// index, -1 for a boundary neighbour (flags only e), -2 for none.
+// index, -1 for a boundary neighbour (flags only e), -2 for none.  With count,
+// zeroes the flag list's count that k_sensor_final appends to.
+//
+// Bound by the FP64 divisions and square roots of the tests, some 1500
+// instructions an element for all four pairs, so a pair first takes bounds of
+// the three measures that need one reciprocal a cell (sensor_quiet) and the
+// tests run only where a bound passes a threshold.  1024x512 two-fluid, three
+// tests on: 20 us against 34 us with every pair tested.
 template <int D, int PH>
-// With init and act (the solver's sensing), the pass also sets init[e] = 0
-// (sensors start at zero, sensor.cc:17-20) and act[e] = 1 (every element
-// active before the first relaxation sweep); with count, zeroes the flag
-// list's count that k_sensor_final appends to.
 __global__ __launch_bounds__(256) void k_sensor_hit(int N_E, int N_N, const int* __restrict__ nb,
                                                     const double* __restrict__ Uavg, SensorTh s,
                                                     int* __restrict__ tgt, int* __restrict__ val,
-                                                    int* __restrict__ init = nullptr, int* __restrict__ act = nullptr,
                                                     int* __restrict__ count = nullptr) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (count && e == 0) *count = 0;
   if (e >= N_E) return;
-  if (init) {
-    init[e] = 0;
-    act[e] = 1;
-  }
-  const SensorCell L = sensor_cell<D, PH>(Uavg, e);
+  const SensorBounds b = sensor_bounds<D, PH>(Uavg, e);
   int t_out = -2, v_out = 0;
-  for (int nn = 0; nn < N_N; nn++) {
-    int right = nb[e * N_N + nn];
-    if (right < 0) { t_out = -1; v_out = 1; break; }
-    const SensorCell R = sensor_cell<D, PH>(Uavg, right);
-    const SensorRoe m = sensor_roe(L, R);
-    if (s.on[0] && sensor_contact(L, R, m, s.th[0])) { t_out = right; v_out = 1; break; }
-    if (s.on[1] && sensor_shock(L, R, m, s.th[1])) { t_out = right; v_out = 2; break; }
-    if (s.on[2] && sensor_gamma(L, R, s.th[2])) { t_out = right; v_out = 3; break; }
+  constexpr int C = 2 * D;  // neighbours whose loads are in flight at once
+  for (int n0 = 0; n0 < N_N && t_out == -2; n0 += C) {
+    int o[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) o[c] = nb[(size_t)e * N_N + min(n0 + c, N_N - 1)];
+    unsigned test = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const SensorBounds r = sensor_bounds<D, PH>(Uavg, o[c] < 0 ? e : o[c]);
+      if (n0 + c < N_N && (o[c] < 0 || !sensor_quiet(b, r, s.on, s.cut))) test |= 1u << c;
+    }
+    if (!test) continue;
+    const SensorCell L = sensor_cell<D, PH>(Uavg, e);
+    for (; test; test &= test - 1) {  // in the neighbours' order
+      const int right = nb[(size_t)e * N_N + n0 + __builtin_ctz(test)];
+      if (right < 0) { t_out = -1; v_out = 1; break; }
+      const SensorCell R = sensor_cell<D, PH>(Uavg, right);
+      const SensorRoe m = sensor_roe(L, R);
+      if (s.on[0] && sensor_contact(L, R, m, s.th[0])) { t_out = right; v_out = 1; break; }
+      if (s.on[1] && sensor_shock(L, R, m, s.th[1])) { t_out = right; v_out = 2; break; }
+      if (s.on[2] && sensor_gamma(L, R, s.th[2])) { t_out = right; v_out = 3; break; }
+    }
   }
   tgt[e] = t_out;
   val[e] = v_out;
 }
 
-// act_in/act_out: 1 if the element runs its tests in the sequential order.
-// prev: the previous sweep's change flag when sweeps are queued in batches;
-// zero there means the fixed point is reached and this sweep does nothing.
-__global__ __launch_bounds__(256) void k_sensor_relax(int N_E, int N_N, const int* __restrict__ nb,
-                                                      const int* __restrict__ init, const int* __restrict__ tgt,
-                                                      const int* __restrict__ act_in, int* __restrict__ act_out,
-                                                      int* __restrict__ changed, const int* prev = nullptr) {
-  if (prev && *prev == 0) return;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= N_E) return;
-  int a = init[e] == 0 ? 1 : 0;
-  if (a) {
-    for (int nn = 0; nn < N_N; ++nn) {
-      int o = nb[e * N_N + nn];
-      if (o >= 0 && o < e && act_in[o] && tgt[o] == e) { a = 0; break; }
+// Whether element x runs its tests in the sequential order: it starts
+// unflagged and no earlier element that runs its tests flags it (tgt == x).
+// The elements that decide it form a tree: each has one target, a later
+// neighbour.  Walked depth first without a stack: down to a pointing
+// neighbour, and back up along the targets.  An element none of whose pointing
+// neighbours runs runs itself and thereby stills its target.
+__device__ inline bool sensor_runs(int x, int N_N, const int* __restrict__ nb, const int* __restrict__ init,
+                                   const int* __restrict__ tgt) {
+  if (init && init[x] != 0) return false;
+  constexpr int C = 4;  // neighbours whose loads are in flight at once
+  int cur = x, nn = 0;
+  for (;;) {
+    int child = -1;
+    for (; nn < N_N && child < 0; nn += C) {
+      int o[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) o[c] = nb[(size_t)cur * N_N + min(nn + c, N_N - 1)];
+#pragma unroll
+      for (int c = C - 1; c >= 0; --c)
+        if (o[c] >= 0 && o[c] < cur && tgt[o[c]] == cur && !(init && init[o[c]] != 0)) child = o[c];
     }
+    if (child >= 0) {
+      cur = child;
+      nn = 0;
+      continue;
+    }
+    // cur runs, so its target p does not; go on with p's target after p
+    if (cur == x) return true;
+    const int p = tgt[cur];
+    if (p == x) return false;
+    cur = tgt[p];
+    for (nn = N_N; nb[(size_t)cur * N_N + nn - 1] != p; --nn) {}
   }
-  act_out[e] = a;
-  if (a != act_in[e]) atomicOr(changed, 1);
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int* p, long n, int v) {
@@ -682,33 +708,52 @@ __global__ __launch_bounds__(256) void k_fill_i32(int* p, long n, int v) {
   if (i < n) p[i] = v;
 }
 
-// last writer in element order wins; untouched elements keep init.  With
-// list, the flagged elements are also appended to list[0 .. *count) (one
-// atomic per block, as k_flag_list; *count zeroed by the hit pass).
-__global__ __launch_bounds__(256) void k_sensor_final(int N_E, int N_N, const int* __restrict__ nb,
-                                                      const int* __restrict__ init, const int* __restrict__ tgt,
-                                                      const int* __restrict__ val, const int* __restrict__ act,
-                                                      int* __restrict__ sensors, int* __restrict__ list = nullptr,
-                                                      int* __restrict__ count = nullptr) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  int bval = 0;
-  if (x < N_E) {
+// The flags of the sequential loop over the elements from their first hits:
+// the last writer in element order wins; untouched elements keep init (zero
+// without it).  With list, the flagged elements are also appended to
+// list[0 .. *count) (one atomic per block; *count zeroed by the hit pass).
+//
+// One pass: each element settles for itself which of the elements that
+// point at it run (sensor_runs), a walk of one or two steps but where long rows
+// of elements point at each other.  The sweeps over the grid it replaces, two
+// to four and one read-back by the host to end them, cost 60 us of launches
+// and 35 us of waiting at 1024x512; it costs 16 us.  Blocks of 1024 elements:
+// their appends to the list are one atomic each on one counter, and with 256
+// elements a block the pass took 25 us.
+constexpr int kFinalBlock = 1024;
+__global__ __launch_bounds__(kFinalBlock) void k_sensor_final(
+    int N_E, int N_N, const int* __restrict__ nb, const int* __restrict__ init, const int* __restrict__ tgt,
+    const int* __restrict__ val, int* __restrict__ sensors, int* __restrict__ list = nullptr,
+    int* __restrict__ count = nullptr) {
+  __shared__ int sN, sBase;
+  __shared__ int sIdx[kFinalBlock];
+  if (threadIdx.x == 0) sN = 0;
+  __syncthreads();
+  const long at = (long)blockIdx.x * kFinalBlock + threadIdx.x;
+  if (at < N_E) {
+    const int x = (int)at;
     int best = -1;
-    bval = init[x];
-    if (act[x] && tgt[x] != -2) { best = x; bval = val[x]; }
-    for (int nn = 0; nn < N_N; ++nn) {
-      int o = nb[x * N_N + nn];
-      if (o >= 0 && act[o] && tgt[o] == x && o > best) { best = o; bval = val[o]; }
+    const int t = tgt[x];
+    int bval = init ? init[x] : 0;
+    constexpr int C = 4;  // neighbours whose loads are in flight at once
+    for (int n0 = 0; n0 < N_N; n0 += C) {
+      int o[C];
+      unsigned points = 0;
+#pragma unroll
+      for (int c = 0; c < C; ++c) o[c] = nb[(size_t)x * N_N + min(n0 + c, N_N - 1)];
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        if (o[c] >= 0 && tgt[o[c]] == x) points |= 1u << c;
+      for (; points; points &= points - 1) {
+        const int q = nb[(size_t)x * N_N + min(n0 + __builtin_ctz(points), N_N - 1)];
+        if (q > best && sensor_runs(q, N_N, nb, init, tgt)) { best = q; bval = val[q]; }
+      }
     }
+    if (t != -2 && x > best && sensor_runs(x, N_N, nb, init, tgt)) bval = val[x];
     sensors[x] = bval;
+    if (list && bval != 0) sIdx[atomicAdd(&sN, 1)] = x;
   }
   if (list) {  // uniform over the launch
-    __shared__ int sN, sBase;
-    __shared__ int sIdx[256];
-    if (threadIdx.x == 0) sN = 0;
-    __syncthreads();
-    const bool f = x < N_E && bval != 0;
-    if (f) sIdx[atomicAdd(&sN, 1)] = x;
     __syncthreads();
     if (threadIdx.x == 0) sBase = sN ? atomicAdd(count, sN) : 0;
     __syncthreads();
@@ -1331,54 +1376,6 @@ hipError_t launch_limit_pr(Solver& s, double* U, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Resolve sequential-order flags from per-element first hits.
-// act_set: the hit pass has already set every element active in s.sens_act.
-static hipError_t sensor_resolve(Solver& s, const int* nb, const int* init, const int* tgt, const int* val,
-                                 int* sensors, hipStream_t st, bool act_set = false, int* list = nullptr,
-                                 int* count = nullptr) {
-  int* act0 = s.sens_act;
-  int* act1 = s.sens_act + s.N_E;
-  if (!act_set) hipLaunchKernelGGL(k_fill_i32, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, act0, (long)s.N_E, 1);
-  // Jacobi sweeps converge to the sequential fixed point after (longest chain + 1) sweeps.
-  if (s.sens_changed) {
-    // batches of kRelaxBatch sweeps with one read-back each: a sweep after one
-    // that changed nothing returns at once (its input already equals its
-    // output, so either buffer holds the fixed point); the batch length is
-    // even, so every batch starts from act0
-    static_assert(kRelaxBatch % 2 == 0, "batches end on act0");
-    for (int it = 0; it <= s.N_E; it += kRelaxBatch) {
-      hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(kRelaxBatch), 0, st, s.sens_changed, (long)kRelaxBatch, 0);
-      for (int i = 0; i < kRelaxBatch; ++i) {
-        hipLaunchKernelGGL(k_sensor_relax, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, s.N_E, s.N_N, nb, init, tgt,
-                           (i % 2) ? act1 : act0, (i % 2) ? act0 : act1, s.sens_changed + i,
-                           i ? s.sens_changed + i - 1 : nullptr);
-      }
-      int h = 0;
-      hipError_t e = hipMemcpyAsync(&h, s.sens_changed + kRelaxBatch - 1, sizeof(int), hipMemcpyDeviceToHost, st);
-      if (e != hipSuccess) return e;
-      if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-      if (!h) break;
-    }
-    hipLaunchKernelGGL(k_sensor_final, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, s.N_E, s.N_N, nb, init, tgt, val,
-                       act0, sensors, list, count);
-    return hipGetLastError();
-  }
-  for (int it = 0; it <= s.N_E; ++it) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(1), 0, st, s.flag, 1L, 0);
-    hipLaunchKernelGGL(k_sensor_relax, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, s.N_E, s.N_N, nb, init, tgt, act0,
-                       act1, s.flag);
-    int h = 0;
-    hipError_t e = hipMemcpyAsync(&h, s.flag, sizeof(int), hipMemcpyDeviceToHost, st);
-    if (e != hipSuccess) return e;
-    if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-    std::swap(act0, act1);
-    if (!h) break;
-  }
-  hipLaunchKernelGGL(k_sensor_final, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, s.N_E, s.N_N, nb, init, tgt, val, act0,
-                     sensors);
-  return hipGetLastError();
-}
-
 hipError_t launch_uavg(const Solver& s, const double* U, double* Uavg, hipStream_t st) {
   const long ncol = (long)s.N_E * s.NF;
   return by_order_ns(s.D, s.P, [&](auto d, auto p) -> hipError_t {
@@ -1388,38 +1385,38 @@ hipError_t launch_uavg(const Solver& s, const double* U, double* Uavg, hipStream
   });
 }
 
+static SensorTh sensor_thresholds(int n, const double* th, const int* on = nullptr) {
+  SensorTh r{};
+  for (int k = 0; k < 3; ++k) {
+    r.on[k] = on ? on[k] : k < n;
+    r.th[k] = th[k];
+    r.cut[k] = sensor_cut(th[k]);
+  }
+  return r;
+}
+
 hipError_t launch_sensing(Solver& s, const double* U, int* sensors, double* Uavg, hipStream_t st, int* list,
                           int* count) {
   if (!Uavg) Uavg = s.Uavg;
-  long ncol = (long)s.N_E * s.NF;
-  hipError_t e = by_order_ns(s.D, s.P, [&](auto d, auto p) -> hipError_t {
-    constexpr int Ns = Shape<decltype(d)::value, decltype(p)::value>::Ns;
-    hipLaunchKernelGGL((k_uavg<Ns>), dim3(nblk(ncol, 256)), dim3(256), 0, st, U, ncol, Uavg);
+  // else the stage kernel that wrote U left its averages in s.Uavg
+  if (s.avgs_of != U || Uavg != s.Uavg) {
+    hipError_t e = launch_uavg(s, U, Uavg, st);
+    if (e != hipSuccess) return e;
+  }
+  const SensorTh th = sensor_thresholds(s.n_thresh, s.thresh);
+  int* tgt = s.sens_tgt;
+  int* val = s.sens_tgt + s.N_E;
+  const dim3 g(nblk(s.N_E, 256)), bl(256);
+  hipError_t e = by_dim_phys(s.D, s.cfg.physics, [&](auto d, auto ph) -> hipError_t {
+    hipLaunchKernelGGL((k_sensor_hit<decltype(d)::value, decltype(ph)::value>), g, bl, 0, st, s.N_E, s.N_N,
+                       s.t.neighbors, Uavg, th, tgt, val, list ? count : nullptr);
     return hipGetLastError();
   });
   if (e != hipSuccess) return e;
-  SensorTh th{};
-  for (int k = 0; k < 3; ++k) { th.on[k] = k < s.n_thresh; th.th[k] = s.thresh[k]; }
-  int* tgt = s.sens_tgt;
-  int* val = s.sens_tgt + s.N_E;
-  // sensors start at zero (sensor.cc:17-20): init, set by the hit pass with the first active set
-  int* init = s.sens_act + 2 * (long)s.N_E;
-  auto hit = [&](auto d, auto ph) -> hipError_t {
-    hipLaunchKernelGGL((k_sensor_hit<decltype(d)::value, decltype(ph)::value>), dim3(nblk(s.N_E, 256)), dim3(256), 0,
-                       st, s.N_E, s.N_N, s.t.neighbors, Uavg, th, tgt, val, init, s.sens_act,
-                       list && s.sens_changed ? count : nullptr);
-    return hipGetLastError();
-  };
-  e = by_dim_phys(s.D, s.cfg.physics, hit);
-  if (e != hipSuccess) return e;
-  if (list && !s.sens_changed) {  // the per-sweep loop below lists nothing: list afterwards
-    hipError_t r = sensor_resolve(s, s.t.neighbors, init, tgt, val, sensors, st, true);
-    if (r != hipSuccess) return r;
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(1), 0, st, count, 1L, 0);
-    hipLaunchKernelGGL(k_flag_list, dim3(nblk(s.N_E, 256)), dim3(256), 0, st, s.N_E, sensors, list, count);
-    return hipGetLastError();
-  }
-  return sensor_resolve(s, s.t.neighbors, init, tgt, val, sensors, st, true, list, count);
+  // sensors start at zero (sensor.cc:17-20)
+  hipLaunchKernelGGL(k_sensor_final, dim3(nblk(s.N_E, kFinalBlock)), dim3(kFinalBlock), 0, st, s.N_E, s.N_N,
+                     s.t.neighbors, nullptr, tgt, val, sensors, list, count);
+  return hipGetLastError();
 }
 
 // One sweep of the flagged HR over the compacted list (see launch_limit_flagged).
@@ -1524,23 +1521,22 @@ hipError_t compat_hrl(int N_s, int N_E, int Nfields, int N_N, int slicenum, cons
 
 hipError_t compat_sensors(Solver& tmp, const int* nb, const double* Uavg, int* sensors, const int* on, const double* th_in,
                           int* scratch) {
-  // scratch: 5*N_E ints: tgt, val, act0, act1, init
-  SensorTh th{};
-  for (int k = 0; k < 3; ++k) { th.on[k] = on[k]; th.th[k] = th_in[k]; }
+  // scratch: 3*N_E ints: tgt, val, init
+  const SensorTh th = sensor_thresholds(3, th_in, on);
   int* tgt = scratch;
   int* val = scratch + tmp.N_E;
-  auto hit = [&](auto d, auto ph) -> hipError_t {
-    hipLaunchKernelGGL((k_sensor_hit<decltype(d)::value, decltype(ph)::value>), dim3(nblk(tmp.N_E, 256)), dim3(256),
-                       0, 0, tmp.N_E, tmp.N_N, nb, Uavg, th, tgt, val);
+  int* init = scratch + 2 * (size_t)tmp.N_E;
+  const dim3 g(nblk(tmp.N_E, 256)), bl(256);
+  hipError_t e = by_dim_phys(tmp.D, tmp.cfg.physics, [&](auto d, auto ph) -> hipError_t {
+    hipLaunchKernelGGL((k_sensor_hit<decltype(d)::value, decltype(ph)::value>), g, bl, 0, 0, tmp.N_E, tmp.N_N, nb,
+                       Uavg, th, tgt, val);
     return hipGetLastError();
-  };
-  hipError_t e = by_dim_phys(tmp.D, tmp.cfg.physics, hit);
+  });
   if (e != hipSuccess) return e;
-  tmp.sens_act = scratch + 2 * tmp.N_E;
-  int* init = scratch + 4 * tmp.N_E;
-  hipError_t ec = hipMemcpyAsync(init, sensors, sizeof(int) * tmp.N_E, hipMemcpyDeviceToDevice, 0);
-  if (ec != hipSuccess) return ec;
-  return sensor_resolve(tmp, nb, init, tgt, val, sensors, 0);
+  if ((e = hipMemcpyAsync(init, sensors, sizeof(int) * tmp.N_E, hipMemcpyDeviceToDevice, 0)) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_sensor_final, dim3(nblk(tmp.N_E, kFinalBlock)), dim3(kFinalBlock), 0, 0, tmp.N_E, tmp.N_N, nb, init,
+                     tgt, val, sensors);
+  return hipGetLastError();
 }
 
 hipError_t compat_hri(int N_s, int N_E, int NF, int N_N, const int* nb, int N_s1D, int slicenum, int offxy, int D,

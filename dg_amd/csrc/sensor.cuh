@@ -131,4 +131,69 @@ __device__ inline bool sensor_gamma(const SensorCell& L, const SensorCell& R, do
   return PHI > th;
 }
 
+// The measures 2x / (1+x)^2 of the three tests rise with x up to x = 1, where
+// they reach 1/2, so a test stays quiet while x is below the smaller root of
+// 2x = th (1+x)^2.  sensor_cut: that root, a thousandth lower for the rounding
+// of both sides, or -1 (never quiet) for thresholds that give no root, or one
+// so small that the thousandth does not cover the rounding.
+__host__ inline double sensor_cut(double th) {
+  if (!(th > 0.0 && th < 0.5)) return -1.0;
+  const double q = 1.0 / th - 1.0, x = 1.0 / (q + sqrt(q * q - 1.0));
+  return x > 1e-6 ? 0.999 * x : -1.0;
+}
+
+// What a cell gives to bounds of the tests' measures; ok: density, alpha,
+// pressure and h = H - v^2/2 are positive and their digits not lost to
+// cancellation (a millionth of what they were subtracted from), so that the
+// bounds hold to 1e-9 of themselves.
+struct SensorBounds {
+  double rho, alpha, p, i, rhoh, h;
+  bool ok;
+};
+
+__device__ inline double fast_rcp(double x) {  // two ulp or so
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+
+template <int D, int PH>
+__device__ inline SensorBounds sensor_bounds(const double* __restrict__ Uavg, int e) {
+  constexpr int NF = Fields<D, PH>::NF;
+  const double* u = Uavg + (size_t)e * NF;
+  SensorBounds b;
+  b.rho = u[0];
+  double m2 = u[1] * u[1];
+  if (D == 2) m2 += u[2] * u[2];
+  const double Et = u[D + 1];
+  b.alpha = (PH == 0 || PH == 2) ? 1 / (kGammaSF - 1) : u[D + 2];
+  const double beta = PH == 3 ? u[D + 3] : 0.0;
+  const double r = fast_rcp(b.rho);
+  const double ke = 0.5 * m2 * r;  // rho v^2 / 2
+  b.i = Et - beta - ke;            // p alpha
+  b.p = b.i * fast_rcp(b.alpha);
+  b.rhoh = Et + b.p - ke;
+  b.h = b.rhoh * r;
+  const double small = 1e-6 * (fabs(Et) + fabs(beta) + ke + fabs(b.p));
+  b.ok = b.rho > 0.0 && b.alpha > 1e-6 && b.alpha < 1e6 && b.p > small && b.i > small && b.rhoh > small;
+  return b;
+}
+
+// True only where none of the tests that are on fires for the pair in either
+// order.  Contact: |dV2| <= |drho| + |dp| / a^2, where a Roe average lies
+// between the cells' values, a^2 >= (gamma-1) min h (the averaged H - v^2/2
+// exceeds the smaller one) and so |dp| / a^2 <= (|di| + max p |dalpha|) / min h.
+// Shock: the pressure jump sensor_shock_w.  Material: the jump of gamma =
+// 1 + 1/alpha, multiplied by both alphas.  A NaN makes a comparison false: the
+// pair is tested.
+__device__ inline bool sensor_quiet(const SensorBounds& l, const SensorBounds& r, const int* on, const double* cut) {
+  if (!(l.ok && r.ok)) return false;
+  const double h = fmin(l.h, r.h), da = fabs(r.alpha - l.alpha);
+  if (on[0] && !(fabs(r.rho - l.rho) * h + fabs(r.i - l.i) + fmax(l.p, r.p) * da <= cut[0] * h * (l.rho + r.rho)))
+    return false;
+  if (on[1] && !(fabs(r.p - l.p) <= cut[1] * (l.p + r.p))) return false;
+  if (on[2] && !(da <= cut[2] * (2.0 * l.alpha * r.alpha + l.alpha + r.alpha))) return false;
+  return true;
+}
+
 }  // namespace dgx

@@ -54,8 +54,8 @@ struct StageArgs {
   double* means;
   const double* __restrict__ w0;
   const double* __restrict__ tensor;  // 2D p=2: 1D tables of vol_tensor_wave
-  double* uavg;   // with means: also the sensor's cell averages [e*5 + f] (sensor_nodal_mean), or null
-  double* psens;  // with uavg: their sensor pressures [e]
+  double* uavg;   // 2D p=2,3 RK stages: the output's sensor averages [e*NF + f] (sensor_nodal_mean), or null
+  double* psens;  // with means and uavg: the averages' sensor pressures [e]
   const int* gate;  // set and nonzero: the launch does nothing (a step skipped by the device-side time control)
 };
 
@@ -916,9 +916,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves
         }
         av[v] = (two ? pre_acc[r * VW + v] : pre_base[r * VW + v]) + gk * du;
         ov[v] = pre_base[r * VW + v] + bk * du;
-        if constexpr (P == 2 && PH == 1) {
-          if (a.means) sU[at] = ov[v];  // this thread's own entry: kept for the cell means below
-        }
+        // this thread's own entry: kept for the cell means and averages below
+        if (PH > 0 && shared_minv && a.uavg) sU[at] = ov[v];
+        if (P == 2 && PH == 1 && shared_minv && a.means) sU[at] = ov[v];
       }
     }
     double* out = (MODE == 0 ? a.fout : a.Uout) + tile0 + off[r];
@@ -962,6 +962,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves
         m[1] = a3[1];
         m[2] = a3[2];
         if (a.uavg) a.psens[eg] = sensor_cell<2, 1>(sA + tid * NF, 0).p;
+      }
+      return;
+    }
+  }
+  if constexpr (MODE == 1 && PH > 0) {
+    if (a.uavg && shared_minv) {  // the sensor's averages alone, one lane per (element, field)
+      __syncthreads();  // the output tile is in sU
+      for (int k = tid; k < NT * NF; k += 256) {
+        const int el = k / NF, f = k % NF;
+        if (in_grid(el * NU))
+          a.uavg[((size_t)(ey0 + el / TX) * a.nx + ex0 + el % TX) * NF + f] = sensor_nodal_mean<Ns>(sU + el * SU + f * Ns);
       }
     }
   }
@@ -1041,6 +1052,12 @@ hipError_t launch_stage_phys(const Solver& s, int mode, int stage, const double*
           a.psens = psens;
           if (means_done) *means_done = true;
         }
+      }
+      // the epilogue's sensor averages alone.  Measured, 1024x512 p = 2
+      // two-fluid: a pass over the state for them takes 34 us, the epilogue 7
+      if (PH > 0 && mode == 1 && !means && uavg && s.t.minv_stride == 0) {
+        a.uavg = uavg;
+        if (means_done) *means_done = true;
       }
       if constexpr (P == 2 && PH <= 1) {
         if (s.precision == 1)
