@@ -421,11 +421,11 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
          upload(s, &s.t.Lag2MonoY, t.Lag2MonoY.data(), t.Lag2MonoY.size()) &&
          upload(s, &s.t.MonoX2Lag, t.MonoX2Lag.data(), t.MonoX2Lag.size());
   s.hr_const = D == 2 && s.P <= 2 && hr_tables_match(s.P, t.Lag2MonoX.data(), t.MonoX2MonoY.data(), t.MonoY2Lag.data());
-  if (s.cart.grid && s.hr_const && s.NF <= 5) {
+  if (s.cart.grid && s.hr_const && s.NF <= 6) {
     // the one-launch HR limiter assumes e -/+ 1 and e -/+ nx inside the grid,
     // takes the rows below and above it and the ends of every row from the
     // table, and takes the x neighbours of a halo-row element to be the halo
-    // elements of the x neighbours (p = 3 would not fit its LDS: two sweeps);
+    // elements of the x neighbours (p <= 2);
     // it carries the three transforms as compile-time constants, so the
     // solver's tables must equal them
     const int nx = s.cart.nx;

@@ -87,7 +87,7 @@ struct Solver {
   bool stage_kernel() const {
     return tiled() || (cart.grid && D == 2 && path != PATH_GENERAL);
   }
-  bool hr2d = false;  // 2D grid whose neighbour table follows it: one-launch HR limiter (k_hr2d)
+  bool hr2d = false;  // 2D grid whose neighbour table follows it: one-launch HR limiter (k_hr2d, k_hr2d_rows)
   bool hr_const = false;  // 2D p <= 2 with the HR transforms of hr_tables.h: constant-table sweeps
   // work buffers
   double* Qe = nullptr;     // face contributions, element-major [((e*N_N+k)*NF+f)*M_s+j]

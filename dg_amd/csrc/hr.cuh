@@ -43,37 +43,58 @@ __device__ inline double integ_deriv_bounds(int k, int n, int a, int b) {
   return ((double)ipow(b, num) - (double)ipow(a, num)) / (double)ifact(num);
 }
 
+// avg[m-1], m = 1..N: the integral over [-1,1] of the (m-1)-th derivative of a
+// slice, all that limit_monomial takes from it
 template <int N>
-__device__ inline void limit_monomial_d(const double* AL, const double* AC, const double* AR, double* Alim) {
+__device__ inline void derivative_averages(const double* A, double* avg) {
 #pragma clang fp contract(off)
-  double avgLC = 0;
 #pragma unroll
-  for (int m = N; m > 0; m--) {
-    double avgdUL = 0, avgdUC = 0, avgdUR = 0, avgRL = 0, avgRC = 0, avgRR = 0;
+  for (int m = 1; m <= N; m++) {
+    double s = 0;
 #pragma unroll
     for (int n = m - 1; n <= N; n++) {
       // the zero integrals (n - m even) are left out: see skip_zero_terms
-      double integral = integ_deriv(m - 1, n);
-      if (integral != 0.0) {
-        avgdUL += AL[n] * integral;
-        avgdUC += AC[n] * integral;
-        avgdUR += AR[n] * integral;
-      }
-      if (n >= m + 1) {
-        double alim = Alim[n];
-        avgRL += alim * integ_deriv_bounds(m - 1, n, -3, -1);
-        if (integral != 0.0) avgRC += alim * integral;
-        avgRR += alim * integ_deriv_bounds(m - 1, n, 1, 3);
-      }
+      const double integral = integ_deriv(m - 1, n);
+      if (integral != 0.0) s += A[n] * integral;
     }
-    double avgLL = 0.5 * (avgdUL - avgRL);
-    avgLC = 0.5 * (avgdUC - avgRC);
-    double avgLR = 0.5 * (avgdUR - avgRR);
+    avg[m - 1] = s;
+  }
+}
+
+// limit_monomial from the averages of the left, own and right slices
+template <int N>
+__device__ inline void limit_averages(const double* L, const double* C, const double* R, double* Alim) {
+#pragma clang fp contract(off)
+  double avgLC = 0;
+#pragma unroll
+  for (int n = 0; n <= N; n++) Alim[n] = 0;
+#pragma unroll
+  for (int m = N; m > 0; m--) {
+    double avgRL = 0, avgRC = 0, avgRR = 0;
+#pragma unroll
+    for (int n = m + 1; n <= N; n++) {
+      const double alim = Alim[n], integral = integ_deriv(m - 1, n);
+      avgRL += alim * integ_deriv_bounds(m - 1, n, -3, -1);
+      if (integral != 0.0) avgRC += alim * integral;
+      avgRR += alim * integ_deriv_bounds(m - 1, n, 1, 3);
+    }
+    double avgLL = 0.5 * (L[m - 1] - avgRL);
+    avgLC = 0.5 * (C[m - 1] - avgRC);
+    double avgLR = 0.5 * (R[m - 1] - avgRR);
     double c1 = 0.5 * (avgLC - avgLL);
     double c2 = 0.5 * (avgLR - avgLC);
     Alim[m] = minmod_d(c1, c2);
   }
   Alim[0] = avgLC;
+}
+
+template <int N>
+__device__ inline void limit_monomial_d(const double* AL, const double* AC, const double* AR, double* Alim) {
+  double L[N], C[N], R[N];
+  derivative_averages<N>(AL, L);
+  derivative_averages<N>(AC, C);
+  derivative_averages<N>(AR, R);
+  limit_averages<N>(L, C, R, Alim);
 }
 
 template <int N>

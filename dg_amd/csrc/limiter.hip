@@ -147,28 +147,67 @@ __device__ inline void col_apply_c(const double* x, double* y) {
   col_apply_c_all<P, WHICH>(x, y, std::make_integer_sequence<int, Ns>{});
 }
 
-// hrl1D for every slice of one column (limiting_kernels.cu:245-319)
+// hrl1D for one slice of a column (limiting_kernels.cu:245-319)
+template <int N>
+__device__ inline void hrl_slice(int physical, int fc, int offxy, const double* AL, const double* AC,
+                                 const double* AR, double* Alim) {
+  if (physical == 2 || (physical == 3 && fc != ((offxy == 0) ? 1 : 2))) {
+    average_monomial_d<N>(AC, Alim);
+  } else if (physical == 3 || physical == 4) {  // wall-normal velocity (3) / gravity tag (4): unchanged
+#pragma unroll
+    for (int n = 0; n <= N; ++n) Alim[n] = AC[n];
+  } else {
+    double lim[N + 1];
+#pragma unroll
+    for (int n = 0; n <= N; ++n) lim[n] = 0.0;
+    limit_monomial_d<N>(AL, AC, AR, lim);
+#pragma unroll
+    for (int n = 0; n <= N; ++n) Alim[n] = lim[n];
+  }
+}
+
+// for every slice of the column
 template <int N, int SL>
 __device__ inline void hrl_column(int physical, int fc, int offxy, const double* AL, const double* AC,
                                   const double* AR, double* Alim) {
-  constexpr int Nsl = N + 1;
 #pragma unroll
   for (int sl = 0; sl < SL; ++sl) {
-    const int o = sl * Nsl;
-    if (physical == 2 || (physical == 3 && fc != ((offxy == 0) ? 1 : 2))) {
-      average_monomial_d<N>(AC + o, Alim + o);
-    } else if (physical == 3 || physical == 4) {  // wall-normal velocity (3) / gravity tag (4): unchanged
-#pragma unroll
-      for (int n = 0; n < Nsl; ++n) Alim[o + n] = AC[o + n];
-    } else {
-      double lim[Nsl];
-#pragma unroll
-      for (int n = 0; n < Nsl; ++n) lim[n] = 0.0;
-      limit_monomial_d<N>(AL + o, AC + o, AR + o, lim);
-#pragma unroll
-      for (int n = 0; n < Nsl; ++n) Alim[o + n] = lim[n];
-    }
+    const int o = sl * (N + 1);
+    hrl_slice<N>(physical, fc, offxy, AL + o, AC + o, AR + o, Alim + o);
   }
+}
+
+template <int P, typename Fn>
+__device__ inline void each_slice(Fn&& fn) {
+  fn(std::integral_constant<int, 0>{});
+  fn(std::integral_constant<int, 1>{});
+  if constexpr (P == 2) fn(std::integral_constant<int, 2>{});
+}
+
+// the rows S*(P+1) .. of col_apply_c: a slice's coefficients
+template <int P, int WHICH, int S, int K>
+__device__ inline void col_apply_c_term(const double* x, double* y) {
+  constexpr int l = K / (P + 1), r = K % (P + 1);
+  constexpr double m = hr_entry<P, WHICH>(S * (P + 1) + r + l * HrTables2D<P>::Ns);
+  if constexpr (l == 0) y[r] = 0.0;
+  if constexpr (m != 0.0) y[r] = y[r] + x[l] * m;
+}
+template <int P, int WHICH, int S, int... K>
+__device__ inline void col_apply_c_slice(const double* x, double* y, std::integer_sequence<int, K...>) {
+  (col_apply_c_term<P, WHICH, S, K>(x, y), ...);
+}
+
+// the columns S*(P+1) .. of col_apply_c: what a slice's coefficients add to y
+template <int P, int WHICH, int S, int... K>
+__device__ inline void col_apply_c_from(const double* x, double* y, std::integer_sequence<int, K...>) {
+  constexpr int Ns = HrTables2D<P>::Ns;
+  auto column = [&](auto k) {
+    constexpr int l = decltype(k)::value;
+    double xs[Ns];
+    xs[S * (P + 1) + l] = x[l];
+    col_apply_c_col<P, WHICH, S*(P + 1) + l>(xs, y, std::make_integer_sequence<int, Ns>{});
+  };
+  (column(std::integral_constant<int, K>{}), ...);
 }
 
 __device__ inline int hr_physical(int left, int right) {
@@ -268,7 +307,8 @@ __global__ __launch_bounds__(256) void k_hr_sweep_c(int N_E, int NF, int N_N, co
 // launches (the products with zero table entries that it leaves out change
 // no finite sum; an Inf or NaN is not spread through its column), and the
 // intermediate state never reaches HBM.  In and Out must differ:
-// neighbouring tiles read In's rows.  At least six waves per SIMD (three
+// neighbouring tiles read In's rows.  For grids of few tiles (see the rule of
+// launch_limit_hr_oop).  At least six waves per SIMD (three
 // 512-thread blocks of the 2D p=2 five-field limiter per CU).
 // RAG: the grid's sides need not be whole tiles; a tile at its right or upper
 // end then holds cols x rows elements, and what lies beyond is absent.
@@ -422,6 +462,205 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6))) void k_
       const int j = q / ROW_OUT, r = q - j * ROW_OUT;
       if (RAG && (j >= rows || r >= cols * EL)) continue;
       Out[((long)(ey0 + j) * nx + ex0) * EL + r] = sA[q];
+    }
+  }
+}
+
+// The same for grids that fill the chip with blocks of many rows each.  Each (element, field) column of a row is limited
+// on its own, with the columns NF before and after it and the rows below and
+// above, so a row is taken as nx*NF columns in a line: a block owns BS of them,
+// one a thread, whatever fields they are, and marches up over H rows.  Per row:
+//   the row's nodal values are in LDS, with NF columns on either side
+//   (coalesced loads, issued a row ahead into registers);
+//   x sweep: a thread forms the Taylor-x coefficients of its column and the two
+//   beside it (Lag2MonoX), limits and turns them to Taylor-y (MonoX2MonoY);
+//   the last three rows' are in its registers;
+//   y sweep of the row below (hrl along y, MonoY2Lag), staged in LDS and
+//   stored as one run of values.
+// The three transforms are the compile-time tables of hr_tables.h, which
+// the host has found equal to the solver's; the ends of the rows and the rows
+// past the grid come from the neighbour table, so periodic ends and walls need
+// no special case (Solver::hr2d says what the table must hold).  Every column
+// of a finite state gets the bits of the two k_hr_sweep launches (the products
+// with zero table entries that it leaves out change no finite sum; an Inf or
+// NaN is not spread through its column), and the intermediate state never
+// reaches HBM.  In and Out must differ: neighbouring blocks read In's rows.
+//
+// Bound by the FP64 additions of the two sweeps (350 a column, exact to the
+// bit, so neither fused nor shared with the columns beside it) as much as by
+// HBM: 1024x512 two-fluid p = 2 takes 110 us, 378 MB in and out at 3.4 TB/s,
+// and 130 us in tiles of 8 x 8, which sweep 1.25 rows a row and form 1.56
+// columns' coefficients a column; 512x256 stiffened p = 2 33 us against 68 us
+// of two sweeps.  What it holds of the last rows are the averages that the y
+// limiter takes from them (6 of 9 numbers) and the slices are kept apart:
+// with all coefficients of three columns and rows in registers it needed 250,
+// or spilled, and took 140 to 340 us.
+template <int P, int NF, int BS>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_hr2d_rows(
+    int nx, int ny, int N_N, int nys, int nblocks, int H, const int* __restrict__ nb, const double* __restrict__ In,
+    double* __restrict__ Out, const int* gate) {
+  if (gate && *gate) return;
+  constexpr int Ns = HrTables2D<P>::Ns, SL = P + 1, TOT = (BS + 2 * NF) * Ns, PER = (TOT + BS - 1) / BS;
+  __shared__ double sIn[TOT], sOut[BS * Ns];
+  // blocks in bands per XCD, upwards first: vertical neighbours share their rows in its L2
+  const int band = (nblocks + 7) / 8, bi = (blockIdx.x % 8) * band + blockIdx.x / 8;
+  if ((int)(blockIdx.x / 8) >= band || bi >= nblocks) return;
+  const int tid = threadIdx.x, NC = nx * NF;
+  const int c0 = (bi / nys) * BS, y0 = (bi % nys) * H, y1 = min(y0 + H, ny);
+  const int ncols = min(BS, NC - c0);
+  const size_t RL = (size_t)NC * Ns;
+  // element in column x of row y, one past the grid on either side, or -1
+  auto elem_at = [&](int y, int x) {
+    const int xx = min(max(x, 0), nx - 1);
+    int e = y < 0 ? nb[(size_t)xx * N_N + 2]
+                  : (y >= ny ? nb[((size_t)(ny - 1) * nx + xx) * N_N + 3] : y * nx + xx);
+    if (x < 0) e = e >= 0 ? nb[(size_t)e * N_N] : -1;
+    if (x >= nx) e = e >= 0 ? nb[(size_t)e * N_N + 1] : -1;
+    return e;
+  };
+  const int c = c0 + min(tid, ncols - 1), ex = c / NF, f = c - ex * NF;
+  const bool endx = ex == 0 || ex == nx - 1;
+  // LDS entry q holds value q of the line from column c0 - NF on; qlo .. qhi lie
+  // in the row, and the element before and the one after it are left to the
+  // first lanes of the blocks at its ends (entry qe)
+  const int qlo = c0 == 0 ? NF * Ns : 0, qhi = min(TOT, (NC - c0 + NF) * Ns);
+  const int xe = tid < NF * Ns ? -1 : nx, qe = xe < 0 ? tid : qhi + tid - NF * Ns;
+  const bool end = tid < 2 * NF * Ns && (xe < 0 ? qlo > 0 : qe < (ncols + 2 * NF) * Ns);
+  static_assert(2 * NF * Ns <= BS, "one lane per value of the row's ends");
+  double pre[PER], pend = 0.0;
+  int px = 0;  // boundary kind along x of this thread's column in the fetched row
+  auto fetch = [&](int y) {
+    if (y >= 0 && y < ny) {
+      const double* row = In + ((size_t)y * RL + (size_t)c0 * Ns);
+      int lo = qlo, hi = qhi - 1;
+      asm volatile("" : "+s"(lo), "+s"(hi));  // the clamped places are not kept in registers from row to row
+#pragma unroll
+      for (int k = 0; k < PER; ++k) pre[k] = row[min(max(tid + k * BS, lo), hi) - NF * Ns];
+      if (end) {
+        const int e = elem_at(y, xe), v = xe < 0 ? tid : tid - NF * Ns;
+        pend = e >= 0 ? In[(size_t)e * NF * Ns + v] : 0.0;
+      }
+    }
+    px = 0;
+    if (endx) {
+      const int e = elem_at(y, ex);
+      if (e >= 0) px = hr_physical(nb[(size_t)e * N_N], nb[(size_t)e * N_N + 1]);
+    }
+  };
+  auto stage = [&](int y) {
+    if (y >= 0 && y < ny) {
+      int lo = qlo, hi = qhi;
+      asm volatile("" : "+s"(lo), "+s"(hi));
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int q = tid + k * BS;
+        if (q >= lo && q < hi) sIn[q] = pre[k];
+      }
+      if (end) sIn[qe] = pend;
+    } else {  // past the grid: column by column through the table
+      for (int w = tid; w < ncols + 2 * NF; w += BS) {
+        const int x = (c0 + w) / NF - 1, e = elem_at(y, x);
+        const double* u = In + ((size_t)max(e, 0) * NF + (c0 + w - (x + 1) * NF)) * Ns;
+#pragma unroll
+        for (int l = 0; l < Ns; ++l) sIn[w * Ns + l] = u[l];
+      }
+    }
+  };
+  using Slice = std::make_integer_sequence<int, P + 1>;
+  using Terms = std::make_integer_sequence<int, Ns*(P + 1)>;
+  // a boundary column: its slice's average or, unchanged, the slice
+  auto boundary = [&](int kind, int un, const double* A, double* Alim) {
+    if (kind == 2 || (kind == 3 && f != un)) {
+      average_monomial_d<P>(A, Alim);
+    } else {
+#pragma unroll
+      for (int n = 0; n <= P; ++n) Alim[n] = A[n];
+    }
+  };
+  double a0[SL * P], a1[SL * P], a2[SL * P];  // derivative_averages along y of rows y-2, y-1, y
+#pragma unroll
+  for (int l = 0; l < SL * P; ++l) a0[l] = a1[l] = 0.0;
+  bool held = false;  // column of row y-1 already stored
+  fetch(y0 - 1);
+  stage(y0 - 1);
+  for (int y = y0 - 1; y <= y1; ++y) {
+    const int physical = px;
+    if (y < y1) fetch(y + 1);
+    __syncthreads();
+    // slice by slice, which the scheduler is kept from mixing: the coefficients
+    // of three columns at once do not fit the registers
+    double t[Ns];
+#pragma unroll
+    for (int l = 0; l < Ns; ++l) t[l] = 0.0;
+    each_slice<P>([&](auto sl) {
+      constexpr int S = decltype(sl)::value;
+      double A[P + 1], L[P], C[P], R[P], Alim[P + 1];
+      col_apply_c_slice<P, 0, S>(sIn + tid * Ns, A, Terms{});
+      derivative_averages<P>(A, L);
+      col_apply_c_slice<P, 0, S>(sIn + (tid + 2 * NF) * Ns, A, Terms{});
+      derivative_averages<P>(A, R);
+      col_apply_c_slice<P, 0, S>(sIn + (tid + NF) * Ns, A, Terms{});
+      derivative_averages<P>(A, C);
+      limit_averages<P>(L, C, R, Alim);
+      if (physical) boundary(physical, 1, A, Alim);
+      col_apply_c_from<P, 1, S>(Alim, t, Slice{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    each_slice<P>([&](auto sl) {
+      constexpr int S = decltype(sl)::value;
+      derivative_averages<P>(t + S * (P + 1), a2 + S * P);
+    });
+    const bool edge = y == 0 || y == ny - 1;
+    if (y > y0 && !held) {
+      double out[Ns];
+#pragma unroll
+      for (int l = 0; l < Ns; ++l) out[l] = 0.0;
+      each_slice<P>([&](auto sl) {
+        constexpr int S = decltype(sl)::value, o = S * P;
+        double Alim[P + 1];
+        limit_averages<P>(a0 + o, a1 + o, a2 + o, Alim);
+        col_apply_c_from<P, 2, S>(Alim, out, Slice{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int l = 0; l < Ns; ++l) sOut[tid * Ns + l] = out[l];
+    }
+    __syncthreads();
+    if (y > y0) {
+      double* o = Out + (size_t)(y - 1) * RL + (size_t)c0 * Ns;
+#pragma unroll
+      for (int k = 0; k < Ns; ++k) {
+        const int q = tid + k * BS;
+        if (q < ncols * Ns) o[q] = sOut[q];
+      }
+    }
+    // rows at the grid's lower and upper end: a boundary column needs no other
+    // row, and its coefficients are at hand only now: staged for the next step
+    held = false;
+    if (edge && y >= y0 && y < y1) {
+      const int* n = nb + ((size_t)y * nx + ex) * N_N;
+      const int kind = hr_physical(n[2], n[3]);
+      __syncthreads();  // sOut is read
+      if (kind) {
+        double out[Ns];
+#pragma unroll
+        for (int l = 0; l < Ns; ++l) out[l] = 0.0;
+        each_slice<P>([&](auto sl) {
+          constexpr int S = decltype(sl)::value;
+          double Alim[P + 1];
+          boundary(kind, 2, t + S * (P + 1), Alim);
+          col_apply_c_from<P, 2, S>(Alim, out, Slice{});
+        });
+#pragma unroll
+        for (int l = 0; l < Ns; ++l) sOut[tid * Ns + l] = out[l];
+        held = true;
+      }
+    }
+    if (y < y1) stage(y + 1);
+#pragma unroll
+    for (int l = 0; l < SL * P; ++l) {
+      a0[l] = a1[l];
+      a1[l] = a2[l];
     }
   }
 }
@@ -1212,7 +1451,7 @@ hipError_t launch_limit_hr(Solver& s, double* U, hipStream_t st) {
   });
 }
 
-// Out = HR(In) with both 2D sweeps in one launch (k_hr2d), p <= 2; needs the
+// Out = HR(In) with both 2D sweeps in one launch, p <= 2; needs the
 // grid layout and a neighbour table that follows it (Solver::hr2d).
 hipError_t launch_limit_hr_oop(Solver& s, const double* In, double* Out, hipStream_t st) {
   if (In == Out) return hipErrorInvalidValue;
@@ -1231,42 +1470,46 @@ hipError_t launch_limit_hr_oop(Solver& s, const double* In, double* Out, hipStre
       return hipGetLastError();
     });
   }
-  if (s.D != 2 || !s.hr2d || (s.NF != 4 && s.NF != 5)) return hipErrorInvalidValue;
-  // 8 x 8 tiles (512 threads) where the rows allow, else 8 x 4: the taller
-  // tile recomputes fewer halo columns (1.56 against 1.88 Taylor-x columns
-  // per output column) and ran 167 against 177 us on the 1024 x 512 p = 2
-  // two-fluid state
-  constexpr int TXE = 8;
-  // grids whose sides are not whole tiles: 8 x 8 ones that reach past the ends
-  const bool ragged = s.cart.nx % TXE != 0 || s.cart.ny % 4 != 0;
-  const int tye = ragged || s.cart.ny % 8 == 0 ? 8 : 4;
-  const int tiles = ((s.cart.nx + TXE - 1) / TXE) * ((s.cart.ny + tye - 1) / tye);
+  if (s.D != 2 || !s.hr2d || s.NF < 4 || s.NF > 6) return hipErrorInvalidValue;
+  constexpr int kStrip = 256, kBlocks = 1024, kTile = 8;  // columns a block, blocks that run at once, tile side
+  const int nx = s.cart.nx, ny = s.cart.ny;
+  const int strips = (nx * s.NF + kStrip - 1) / kStrip;
+  // Marching pays once the rows of all strips are more than the chip takes at a
+  // time: then a block has two or more, else only its three dependent rows.
+  // Measured, rows against tiles (with some 8 us of launch): two-fluid p = 2
+  // 256x128 22 against 17 us, 384x192 31 against 30, 512x512 65 against 76,
+  // 1024x512 120 against 140, 2048x1024 408 against 548.  More than six rows a
+  // block no longer pay for fewer blocks in flight (1024x512: 120 us with 6,
+  // 125 with 8, 129 with 11).
+  const bool rows = 2L * strips * ny > 3 * kBlocks;
   return by_order_ns(s.D, s.P, [&](auto d, auto p) -> hipError_t {
     constexpr int D = decltype(d)::value, P = decltype(p)::value;
     if constexpr (D == 2 && P <= 2) {
       constexpr int Ns = Shape<D, P>::Ns, SL = P + 1;
-      auto go = [&](auto nf, auto ty) -> hipError_t {
-        constexpr int NF = decltype(nf)::value, TYE = decltype(ty)::value, BS = TYE == 4 ? 256 : 512;
-        const bool vec = (reinterpret_cast<uintptr_t>(Out) & 15) == 0;
+      auto go = [&](auto nf) -> hipError_t {
+        constexpr int NF = decltype(nf)::value;
+        if (rows) {
+          const int H = std::min(6, (int)((long)strips * ny / kBlocks) + 1), nys = (ny + H - 1) / H, nblocks = strips * nys;
+          hipLaunchKernelGGL((k_hr2d_rows<P, NF, kStrip>), dim3(8 * ((nblocks + 7) / 8)), dim3(kStrip), 0, st, nx, ny,
+                             s.N_N, nys, nblocks, H, s.t.neighbors, In, Out, s.gate);
+          return hipGetLastError();
+        }
+        const bool ragged = nx % kTile != 0 || ny % kTile != 0;
+        const bool vec = (reinterpret_cast<uintptr_t>(Out) & 15) == 0 && (!ragged || NF * Ns % 2 == 0 || nx % 2 == 0);
+        const dim3 tiles(((nx + kTile - 1) / kTile) * ((ny + kTile - 1) / kTile));
         auto run = [&](auto kern) {
-          hipLaunchKernelGGL(kern, dim3(tiles), dim3(BS), 0, st, s.cart.nx, s.cart.ny, s.N_N, s.t.neighbors, In, Out,
-                             s.gate);
+          hipLaunchKernelGGL(kern, tiles, dim3(512), 0, st, nx, ny, s.N_N, s.t.neighbors, In, Out, s.gate);
           return hipGetLastError();
         };
-        if constexpr (TYE == 8) {
-          if (ragged)
-            return vec && (NF * Ns % 2 == 0 || s.cart.nx % 2 == 0)
-                       ? run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, true, true>)
-                       : run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, false, true>);
-        }
-        return vec ? run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, true, false>)
-                   : run(k_hr2d<Ns, P, SL, NF, TXE, TYE, BS, false, false>);
+        if (ragged)
+          return vec ? run(k_hr2d<Ns, P, SL, NF, kTile, kTile, 512, true, true>)
+                     : run(k_hr2d<Ns, P, SL, NF, kTile, kTile, 512, false, true>);
+        return vec ? run(k_hr2d<Ns, P, SL, NF, kTile, kTile, 512, true, false>)
+                   : run(k_hr2d<Ns, P, SL, NF, kTile, kTile, 512, false, false>);
       };
-      using I4 = std::integral_constant<int, 4>;
-      using I5 = std::integral_constant<int, 5>;
-      using I8 = std::integral_constant<int, 8>;
-      if (s.NF == 4) return tye == 8 ? go(I4{}, I8{}) : go(I4{}, I4{});
-      return tye == 8 ? go(I5{}, I8{}) : go(I5{}, I4{});
+      if (s.NF == 4) return go(std::integral_constant<int, 4>{});
+      if (s.NF == 5) return go(std::integral_constant<int, 5>{});
+      return go(std::integral_constant<int, 6>{});
     }
     return hipErrorInvalidValue;
   });
