@@ -601,8 +601,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves
   __shared__ __align__(16) double sW[NFACE * MG * NWP];  // face-point fluxes
   // TENSOR: the 1D tables; else the reference tables until every wave has taken
   // its operands, then the element phases' flux rows
-  constexpr int O_DW = V::NTAB_PHI, O_MINV = O_DW + V::NTAB_D, O_DPHI = O_MINV + Ns * Ns,
-                O_PW = O_DPHI + (NNC ? V::NTAB_D : 0), NTAB = O_PW + (NNC ? V::NTAB_PHI : 0);
+  constexpr int LDD = VolOps<TW, P, PH>::LDD, LDP = VolOps<TW, P, PH>::LDP, NG = V::NG;
+  constexpr int O_DW = V::NTAB_PHI, O_MINV = O_DW + Ns * LDD, O_DPHI = O_MINV + Ns * Ns,
+                O_PW = O_DPHI + (NNC ? V::NTAB_D : 0), NTAB = O_PW + (NNC ? Ns * LDP : 0);
   constexpr int NFLUX = 4 * vol_wave_flux<TW, P>(), NFT = NTAB > NFLUX ? NTAB : NFLUX;
   __shared__ double sFlux[TENSOR ? kTensorTables * 16 : NFT];
   __shared__ double sPsi[MG * Ms], sPsiw[MG * Ms];
@@ -764,14 +765,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves
 #pragma unroll
   for (int r = 0; r < R_D; ++r)
     if (tid + r * 256 < V::NTAB_D) {
-      sFlux[O_DW + tid + r * 256] = tdw[r];
+      const int k = tid + r * 256;
+      sFlux[O_DW + k / (2 * NG) * LDD + k % (2 * NG)] = tdw[r];
       if constexpr (NNC > 0) sFlux[O_DPHI + tid + r * 256] = tdphi[r];
     }
 #pragma unroll
   for (int r = 0; r < R_T; ++r)
     if (tid + r * 256 < V::NTAB_PHI) {
       sFlux[tid + r * 256] = tphi[r];
-      if constexpr (NNC > 0) sFlux[O_PW + tid + r * 256] = tpw[r];
+      const int k = tid + r * 256;
+      if constexpr (NNC > 0) sFlux[O_PW + k / NG * LDP + k % NG] = tpw[r];
     }
   if (tid < Ns * Ns) sFlux[O_MINV + tid] = tminv;
   }

@@ -328,6 +328,10 @@ constexpr int vol_wave_extra() { return VolMfma<P, PH>::NSR * 8 * VolMfma<P, PH>
 template <typename T, int P, int PH, typename TM = T>
 struct VolOps {
   using M = VolMfma<P, PH>;
+  // row strides of dphi_w and phi_w in LDS: lanes read along a column, which at
+  // NG = 16 would lie in one bank (p = 2 with FP32 contractions, two-fluid
+  // 1024x512 without limiter: 966 us a step unpadded, 935 so)
+  static constexpr int LDD = 2 * M::NG + (M::NG % 16 == 0), LDP = M::NG + (M::NG % 16 == 0);
   TM phi[M::CB][M::KN];
   T dw[2][M::KG];
   double minv[M::KN];
@@ -363,8 +367,8 @@ struct VolOps {
       const int g = 4 * s + q;
       const bool in = (NG % 4 == 0 || g < NG) && (Ns == 16 || c < Ns);
 #pragma unroll
-      for (int al = 0; al < 2; ++al) dw[al][s] = (T)at(dphi_w, in, c * NG * 2 + g * 2 + al);
-      if constexpr (M::NNC > 0) pw[s] = at(phi_w, in, g + c * NG);
+      for (int al = 0; al < 2; ++al) dw[al][s] = (T)at(dphi_w, in, c * LDD + g * 2 + al);
+      if constexpr (M::NNC > 0) pw[s] = at(phi_w, in, g + c * LDP);
     }
   }
 };
