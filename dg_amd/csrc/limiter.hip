@@ -1494,6 +1494,17 @@ hipError_t launch_limit_hr_oop(Solver& s, const double* In, double* Out, hipStre
                              s.N_N, nys, nblocks, H, s.t.neighbors, In, Out, s.gate);
           return hipGetLastError();
         }
+        if constexpr (NF <= 5) {  // rows of 8 x 4 tiles (256 threads): twice the blocks of ragged 8 x 8 ones
+          if (nx % kTile == 0 && ny % 8 == 4) {
+            auto run = [&](auto kern) {
+              hipLaunchKernelGGL(kern, dim3((nx / kTile) * (ny / 4)), dim3(256), 0, st, nx, ny, s.N_N, s.t.neighbors,
+                                 In, Out, s.gate);
+              return hipGetLastError();
+            };
+            return (reinterpret_cast<uintptr_t>(Out) & 15) == 0 ? run(k_hr2d<Ns, P, SL, NF, kTile, 4, 256, true, false>)
+                                                                : run(k_hr2d<Ns, P, SL, NF, kTile, 4, 256, false, false>);
+          }
+        }
         const bool ragged = nx % kTile != 0 || ny % kTile != 0;
         const bool vec = (reinterpret_cast<uintptr_t>(Out) & 15) == 0 && (!ragged || NF * Ns % 2 == 0 || nx % 2 == 0);
         const dim3 tiles(((nx + kTile - 1) / kTile) * ((ny + kTile - 1) / kTile));
