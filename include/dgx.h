@@ -138,7 +138,7 @@ void Lcopy_detected(int N_s, int N_E, int* sensors, double* Uold, double* U);
 /* No counterpart in the reference: Lcalc_sensors for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc).  Same arguments and flags as
- * Lcalc_sensors; its scratch is a fixed per-device array (40 MiB) instead of
+ * Lcalc_sensors; its scratch is a fixed per-device array (24 MiB) instead of
  * hipMalloc, so N_E is limited to 2^21 elements (DGX_EINVAL beyond, with
  * dgx_last_error()).  Calls that overlap on one GPU share that array and race.
  * Synchronous, null stream, like the reference launchers. */
