@@ -589,8 +589,8 @@ __device__ inline void node_edges(int c, int* edge, int* pos) {
 // loads and the output.
 //
 // Bound by HBM and by how much of a block's serial chain the other blocks of
-// its CU hide.  1024x512 two-fluid, p = 2: 212 us a launch (755 MB of states,
-// 925 MB measured: 4.4 TB/s of the 4.9 a copy reaches) against 309 us of the
+// its CU hide.  1024x512 two-fluid, p = 2: 214 us a launch (755 MB of states,
+// 901 MB measured: 4.2 TB/s of the 4.9 a copy reaches) against 309 us of the
 // kernel before it, which summed the faces into per-element edges behind a
 // barrier of its own, kept the reference tables in LDS (50.8 KB, three blocks
 // a CU; now 30.5 KB and four) and ran 28 16x16x4 products and the fields after
