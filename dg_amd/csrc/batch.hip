@@ -56,7 +56,7 @@ struct BatchArgs {
   double* Out;              // null: only the maxima
   double* T;                // [problem] accumulated time
   int* status;              // [problem] 0 ok, 1 Dt too small or NaN
-  const double* part_in;    // [workgroup] maxima of |u|+a
+  const double* part_in;    // [workgroup] maxima of |u|+a; NaN: the problem has stopped
   double* part_out;
   double cfl;               // the deck's CFL number
   int limiter, stages;      // stages 0: only the limiter, and the maxima
@@ -86,21 +86,28 @@ __device__ __forceinline__ void batch_segment(const BatchArgs& a, const BatchSeg
   const long so = a.state_off[pid], eo = a.elem_off[pid];
   const double* In = a.In + so;
   double* Out = a.Out ? a.Out + so : nullptr;
-  bool stopped = a.status[pid] != 0;
+  // Whether the problem has stopped.  Every thread of its workgroups must come
+  // to the same answer, since barriers follow: a run's first launch takes it
+  // from the caller's status, which no launch of that kind writes; the steps
+  // take it from the maxima alone, of which a stopped segment leaves a NaN.
+  bool stopped;
   double dt = 0.0;
-  if (!stopped && a.stages) {
+  if (a.stages) {
     double v = 0.0;
     for (int k = tid; k < sg.n; k += nthr) v = nanmax(v, a.part_in[sg.wg0 + k]);
     dt = a.cfl * a.dx[pid] / (2 * P + 1) / block_nanmax(v, red);  // main.cc:896-897, rk.cc:268
     stopped = !(dt >= 1e-14);
-    if (tid == 0 && sg.c0 == 0) {
-      if (stopped) a.status[pid] = 1;
-      else a.T[pid] = a.T[pid] + dt;
+    if (tid == 0 && sg.c0 == 0) {  // the only thread that reads or writes the problem's status in a step
+      if (!stopped) a.T[pid] = a.T[pid] + dt;
+      else if (a.status[pid] == 0) a.status[pid] = 1;
     }
+  } else {
+    stopped = a.status[pid] != 0;
   }
   if (stopped) {  // the state moves on as it is
     if (Out)
       for (long k = (long)sg.c0 * NU + tid; k < (long)sg.c1 * NU; k += nthr) Out[k] = In[k];
+    if (tid == 0) a.part_out[blockIdx.x] = __builtin_nan("");
     return;
   }
   Tab1D t = a.tab[P - 1];
