@@ -912,25 +912,27 @@ __global__ __launch_bounds__(256) void k_sensor_hit(int N_E, int N_N, const int*
 // The elements that decide it form a tree: each has one target, a later
 // neighbour.  Walked depth first without a stack: down to a pointing
 // neighbour, and back up along the targets.  An element none of whose pointing
-// neighbours runs runs itself and thereby stills its target.
+// neighbours runs runs itself and thereby stills its target.  The neighbours
+// that point at an element are taken in the order of their numbers, whatever
+// their places in the table: one that is listed twice is visited once.
 __device__ inline bool sensor_runs(int x, int N_N, const int* __restrict__ nb, const int* __restrict__ init,
                                    const int* __restrict__ tgt) {
   if (init && init[x] != 0) return false;
   constexpr int C = 4;  // neighbours whose loads are in flight at once
-  int cur = x, nn = 0;
+  int cur = x, after = -1;
   for (;;) {
-    int child = -1;
-    for (; nn < N_N && child < 0; nn += C) {
+    int child = cur;
+    for (int nn = 0; nn < N_N; nn += C) {
       int o[C];
 #pragma unroll
       for (int c = 0; c < C; ++c) o[c] = nb[(size_t)cur * N_N + min(nn + c, N_N - 1)];
 #pragma unroll
-      for (int c = C - 1; c >= 0; --c)
-        if (o[c] >= 0 && o[c] < cur && tgt[o[c]] == cur && !(init && init[o[c]] != 0)) child = o[c];
+      for (int c = 0; c < C; ++c)
+        if (o[c] > after && o[c] < cur && tgt[o[c]] == cur && !(init && init[o[c]] != 0)) child = min(child, o[c]);
     }
-    if (child >= 0) {
+    if (child != cur) {
       cur = child;
-      nn = 0;
+      after = -1;
       continue;
     }
     // cur runs, so its target p does not; go on with p's target after p
@@ -938,7 +940,7 @@ __device__ inline bool sensor_runs(int x, int N_N, const int* __restrict__ nb, c
     const int p = tgt[cur];
     if (p == x) return false;
     cur = tgt[p];
-    for (nn = N_N; nb[(size_t)cur * N_N + nn - 1] != p; --nn) {}
+    after = p;
   }
 }
 
@@ -956,7 +958,9 @@ __global__ __launch_bounds__(256) void k_fill_i32(int* p, long n, int v) {
 // point at it run (sensor_runs), a walk of one or two steps but where long rows
 // of elements point at each other.  The sweeps over the grid it replaces, two
 // to four and one read-back by the host to end them, cost 60 us of launches
-// and 35 us of waiting at 1024x512; it costs 16 us.  Blocks of 1024 elements:
+// and 35 us of waiting at 1024x512; it costs 16 us.  A row of n elements that
+// all point at the next one is n dependent steps for its last element, and was
+// n sweeps: 1000 elements 1.4 ms against 8.5, 64000 elements 107 against 870.  Blocks of 1024 elements:
 // their appends to the list are one atomic each on one counter, and with 256
 // elements a block the pass took 25 us.
 constexpr int kFinalBlock = 1024;
