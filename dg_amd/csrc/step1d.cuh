@@ -148,16 +148,17 @@ __device__ __forceinline__ void window_limit(const Tab1D& t, const Mesh1D& m, in
 // One RK4 step (stages == 4) or only a limiter application (stages == 0) of
 // the owned elements [c0, c1), In -> Out (element-major states of the whole
 // problem; In != Out; a null Out: only umax).  The window, [c0, c1) and its
-// halo, may not exceed W elements, a multiple of R; the halo is cut at the ends of a problem that
-// is not periodic.  get_dt(dt) is called once by every thread, the window's
-// loads in flight, and gives the step's Dt (it may synchronise the block); the
-// step is left out when it returns false.  umax(u, e, q) is called with the
-// fields of every owned node of the new state.  Every thread of the block
+// halo, may not exceed W elements, a multiple of R; the halo is cut at the ends
+// of a problem that is not periodic.  get_dt(dt) is called once by every thread,
+// the window's loads in flight, and gives the step's Dt (it may synchronise the
+// block); when it returns false the step is left out and step_window returns
+// false.  umax(u, e, q) is called with the fields of every owned node of the new
+// state.  Every thread of the block
 // calls it (a multiple of 64 threads, W/R*N_s of them with nodes); LS =
 // row_1d of W or more, lds holds 6*N_s*N_s + LS*(2*N_F*N_s + N_F + NNC)
 // doubles.
 template <int P, int PH, int FL, int R, int LS, typename GetDt, typename UMax>
-__device__ __forceinline__ void step_window(const Tab1D& t, const Mesh1D& m, int c0, int c1, const double* In,
+__device__ __forceinline__ bool step_window(const Tab1D& t, const Mesh1D& m, int c0, int c1, const double* In,
                                             double* Out, GetDt&& get_dt, bool limited, int stages, double* lds,
                                             int W, UMax&& umax) {
   using V = Vol<1, P, PH>;
@@ -218,7 +219,7 @@ __device__ __forceinline__ void step_window(const Tab1D& t, const Mesh1D& m, int
     sT[k] = x;
   }
   double dt = 0.0;
-  if (!get_dt(dt)) return;
+  if (!get_dt(dt)) return false;
 #pragma unroll
   for (int k = 0; k < KL; ++k) {
     const int i = tid + k * nthr;
@@ -396,6 +397,7 @@ __device__ __forceinline__ void step_window(const Tab1D& t, const Mesh1D& m, int
       for (int f = 0; f < NF; ++f) u[f] = A[(f * Ns + q) * LS + e[r]];
       umax(u, w0 + e[r], q);
     }
+  return true;
 }
 
 }  // namespace dgx

@@ -96,14 +96,15 @@ __global__ __launch_bounds__(256) void k_step1d(Step1DArgs a) {
   };
   const int c0 = blockIdx.x * a.own, c1 = min(a.m.NE, c0 + a.own);
   double v = 0.0;
-  step_window<P, PH, FL, R, row_1d(window_1d(LANES, R, P))>(a.t, a.m, c0, c1, a.In, a.Out, get_dt, a.limited != 0, a.stages, lds,
-                            window_1d(LANES, R, P), [&](const double* u, int e, int q) {
-                              if (!a.part_out) return;
-                              const double s = upa<1, PH>(u);
-                              if (e == 0 && q == 0) a.part_out[gridDim.x] = s;
-                              v = skip_nan(v, s);
-                            });
-  if (a.part_out) {  // not reached by a step that was left out
+  const bool taken = step_window<P, PH, FL, R, row_1d(window_1d(LANES, R, P))>(
+      a.t, a.m, c0, c1, a.In, a.Out, get_dt, a.limited != 0, a.stages, lds, window_1d(LANES, R, P),
+      [&](const double* u, int e, int q) {
+        if (!a.part_out) return;
+        const double s = upa<1, PH>(u);
+        if (e == 0 && q == 0) a.part_out[gridDim.x] = s;
+        v = skip_nan(v, s);
+      });
+  if (taken && a.part_out) {  // the same for every thread; a step that was left out leaves no maxima
     const double mx = block_skip_nan(v, red_out);
     if (tid == 0) a.part_out[blockIdx.x] = mx;
   }
