@@ -351,7 +351,8 @@ class Solver:
         _check(lib().dgx_conservation(self._h, self._u(U), _ptr(totals), _stream(stream)), "dgx_conservation")
 
     def set_path(self, path: int) -> None:
-        """PATH_AUTO, PATH_GENERAL (face + element kernels) or PATH_TILED (one fused kernel per stage)."""
+        """PATH_AUTO (the fused kernels wherever the mesh is a grid), PATH_GENERAL (face + element kernels) or
+        PATH_TILED (as PATH_AUTO, refused unless the mesh is a built grid of whole tiles)."""
         _check(lib().dgx_solver_set_path(self._h, path), "dgx_solver_set_path")
 
     def set_precision(self, precision: int) -> None:
@@ -361,7 +362,8 @@ class Solver:
 
     @property
     def path(self) -> int:
-        """Kernel path in use: PATH_GENERAL or PATH_TILED."""
+        """PATH_TILED on built grids of whole tiles unless PATH_GENERAL is set, else PATH_GENERAL.  Ragged grids and
+        Gmsh files in grid order report PATH_GENERAL and run the tile kernel too (profile_read counts launches)."""
         return lib().dgx_solver_path(self._h)
 
     @property

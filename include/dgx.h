@@ -234,13 +234,19 @@ dgx_status dgx_rk4_integrate_out(dgx_solver* s, double* U, double cfl, const dou
                                  int limiter, dgx_output_fn on_output, void* user, int* steps, double* t_final,
                                  void* stream);
 
-/* Kernel path.  0 auto: the fused tile kernel (one launch per RK stage)
- * on uniform Cartesian meshes whose element counts are multiples of the tile
- * (8x4 elements in 2D, 128 in 1D), else the face + element kernels;
- * 1 face + element kernels; 2 tile kernel (DGX_EUNSUPPORTED when the mesh
- * does not qualify).  Both paths compute the same right-hand side as
- * DG_SOLVER::dg_solver (dg_solver.h:292-364).  dgx_solver_path reports the
- * path in use (1 or 2). */
+/* Kernel path.  0 auto: one fused kernel per RK stage (the tile kernel) on 2D
+ * grids of any size, built or read from a file whose elements are in grid
+ * order; in 1D one kernel per RK4 step with limiters 0 and 1, and the tile
+ * kernel otherwise on built meshes of whole tiles; elsewhere the face + element
+ * kernels.  1: face + element kernels.  2: as 0, refused with DGX_EUNSUPPORTED
+ * unless the mesh was built as a Cartesian grid whose sides are whole tiles
+ * (8x4 elements in 2D, 8 in 1D), the grids on which the tile kernel also has the
+ * reduced precisions below.  Every path computes the same right-hand
+ * side of DG_SOLVER::dg_solver (dg_solver.h:292-364).
+ * dgx_solver_path tells which kind of grid the solver has under its present
+ * path: 2 on such whole-tile grids unless path 1 is set, else 1.  It does not
+ * name the kernel that runs: ragged grids and files in grid order report 1 and
+ * run the tile kernel too (dgx_profile_read counts the launches of each). */
 dgx_status dgx_solver_set_path(dgx_solver* s, int path);
 /* Precision of the tile kernel's volume contractions: 0 FP64 (default);
  * 1 the map to the Gauss points and the integration against the test
