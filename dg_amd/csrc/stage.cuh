@@ -606,8 +606,11 @@ __device__ inline void node_edges(int c, int* edge, int* pos) {
 // 16-byte pairs (every state pointer and row start is 16-byte aligned and,
 // with RAG, every row of a tile a whole number of pairs, which the host checks
 // before it picks this instance).  RAG: the grid's sides need not be whole
-// tiles; the tile's elements past its ends repeat the tile's first element and
-// are not stored.
+// tiles; the tile's elements past its ends hold values of its first element, in
+// its order or, where pairs of an odd number of values an element keep it out,
+// shifted (not a state then, so anything may come of them).  They are not
+// stored, and nothing of the grid's own elements depends on them: a face past
+// the ends contributes nowhere and a row of a matrix product is one element's.
 // Waves per SIMD the registers must allow.  Measured, us a step without
 // limiter: p = 2 single fluid 512x512 353 with 4 and 5, 473 with 6 (spills);
 // two-fluid 1024x512 849 with 3 and 4, 917 with 5; stiffened 512x256 315 with 3
@@ -683,7 +686,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves
     off[r] = offset(k);
     if (k < NT * NU) {
       unsigned o = off[r];
-      if constexpr (RAG) {
+      if constexpr (RAG) {  // an aligned pair of the first element (k is even)
         if (!in_grid(k)) o = VEC && NU % 2 ? k % (NU - 1) : k % NU;
       }
       const double* src = a.Uin + tile0 + o;
