@@ -287,24 +287,26 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs a) {
   if (tid < MG * Ms) { psi_r = a.psi[tid]; psiw_r = a.psi_w[tid]; }
   const double dt = (MODE == 1) ? a.dt[0] : 0.0;
   const int ex0 = (tile % a.tiles_x) * TX, ey0 = (tile / a.tiles_x) * TY;
+  // Lanes past the tile's entries read its last ones: under a condition the
+  // pairs of both rounds became one value, whose copy waited for the first load
+  // before any other was issued (a launch of two-fluid 64x32 7.9 us, 7.55 so;
+  // 200x100 11.95 and 11.65).
   double pu[R_U * VW], ph[R_H], pg[R_G], pf[R_F];
 #pragma unroll
   for (int r = 0; r < R_U; ++r) {
-    const int k = VW * (tid + r * 256);
-    if (k < NT * NU) {
-      const int ty = k / (TX * NU);
-      const double* src = a.Uin + ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
-      if constexpr (RAG) {
-        if (ey0 + ty >= a.ny || k - ty * TX * NU >= (a.nx - ex0) * NU)
-          src = a.Uin + ((size_t)ey0 * a.nx + ex0) * NU + k % NU;
-      }
-      if constexpr (VEC) {
-        const double2 v = *reinterpret_cast<const double2*>(src);
-        pu[2 * r] = v.x;
-        pu[2 * r + 1] = v.y;
-      } else {
-        pu[r] = *src;
-      }
+    const int k = min(VW * (tid + r * 256), NT * NU - VW);
+    const int ty = k / (TX * NU);
+    const double* src = a.Uin + ((size_t)(ey0 + ty) * a.nx + ex0) * NU + (k - ty * TX * NU);
+    if constexpr (RAG) {
+      if (ey0 + ty >= a.ny || k - ty * TX * NU >= (a.nx - ex0) * NU)
+        src = a.Uin + ((size_t)ey0 * a.nx + ex0) * NU + k % NU;
+    }
+    if constexpr (VEC) {
+      const double2 v = *reinterpret_cast<const double2*>(src);
+      pu[2 * r] = v.x;
+      pu[2 * r + 1] = v.y;
+    } else {
+      pu[r] = *src;
     }
   }
 #pragma unroll
