@@ -161,14 +161,24 @@ static hipError_t dispatch_batch(const dgx_config& c, Fn&& fn) {
 }
 
 // Elements per lane by workgroup size: three, and registers for two waves per
-// SIMD, up to 128 threads; two and three waves up to 256; one and four above.
+// SIMD (one where the launch has no more, kLoneWaves), up to 128 threads; two and
+// three waves up to 256; one and four above.
 // A segment is cut to no less than 64 elements, which at order 3 and 128
-// threads takes one window of three elements a lane and two of two: 16 problems
+// threads takes one window of three elements a lane and two of two (all with
+// registers for two waves per SIMD): 16 problems
 // of up to 400 elements 66 us a step against 80, 48 of 2000 53 against 70, 256
 // of 4000 239 against 244 (four and two 349, one and four 316).  256 threads 197
 // (one and four 248, three and two 229), 512 threads 207 (two waves 302), 1024
 // threads 230.
 static int batch_R(int block) { return block <= 128 ? 3 : (block <= 256 ? 2 : 1); }
+// Waves of a launch up to which workgroups of up to 128 threads take the
+// instance for one wave per SIMD (262 registers, no spills; the other is held to
+// 256, spills and has less room to reorder): the card has 1024 SIMDs, so no wave
+// has to share one.  us a step with the two forced: 16 problems
+// of up to 400 elements (34 workgroups) 58 against 66, 150 of 600 (500) 60
+// against 68, 48 of 2000 (441) 40 against 52; past the line 64 of 2000 (581) 71
+// against 69, 128 of 2000 (1221) 109 against 85.
+constexpr int kLoneWaves = 1024;
 // The launch bound of the instance that runs workgroups of `block` threads.
 static int batch_LB(int block) { return block <= 128 ? 128 : (block <= 256 ? 256 : (block <= 512 ? 512 : 1024)); }
 
@@ -295,7 +305,8 @@ hipError_t launch_batch(dgx_batch* b, int block, const double* In, double* Out, 
   return dispatch_batch(b->cfg, [&](auto ph, auto fl) -> hipError_t {
     constexpr int PH = decltype(ph)::value, FL = decltype(fl)::value;
     const dim3 g(b->G), t(block);
-    if (LB == 128) hipLaunchKernelGGL((k_batch<PH, FL, 3, 128, 2>), g, t, lds, st, a);
+    if (LB == 128 && b->G * (block / 64) <= kLoneWaves) hipLaunchKernelGGL((k_batch<PH, FL, 3, 128, 1>), g, t, lds, st, a);
+    else if (LB == 128) hipLaunchKernelGGL((k_batch<PH, FL, 3, 128, 2>), g, t, lds, st, a);
     else if (LB == 256) hipLaunchKernelGGL((k_batch<PH, FL, 2, 256, 3>), g, t, lds, st, a);
     else if (LB == 512) hipLaunchKernelGGL((k_batch<PH, FL, 1, 512, 4>), g, t, lds, st, a);
     else hipLaunchKernelGGL((k_batch<PH, FL, 1, 1024, 4>), g, t, lds, st, a);
