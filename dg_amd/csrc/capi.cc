@@ -447,7 +447,7 @@ dgx_status dgx_solver_create(const dgx_config* cfg, const dgx_mesh* mesh, dgx_so
   }
   const size_t S = (size_t)s.state_size();
   ok = ok && alloc(s, &s.Qe, (size_t)NE * NN * s.NF * s.M_s) && alloc(s, &s.Uacc, S) && alloc(s, &s.Ustar, S) &&
-       alloc(s, &s.work, S) && alloc(s, &s.work2, S) && alloc(s, &s.Uavg, (size_t)NE * s.NF) &&
+       alloc(s, &s.work, S) && alloc(s, &s.Uavg, (size_t)NE * s.NF) &&
        alloc(s, &s.sensors, (size_t)NE) && alloc(s, &s.sens_tgt, (size_t)2 * NE) &&
        alloc(s, &s.flag, 4) && alloc(s, &s.flag_list, (size_t)NE) &&
        alloc(s, &s.dscratch, 8) && alloc(s, &s.time_state, 8) &&

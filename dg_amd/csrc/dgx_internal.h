@@ -95,7 +95,6 @@ struct Solver {
   double* Ustar = nullptr;  // stage state
   double* Ustar2 = nullptr; // second stage state (tile path, see rk4_step)
   double* work = nullptr;   // limiter scratch (state size)
-  double* work2 = nullptr;  // limiter scratch (state size)
   double* Uavg = nullptr;   // [e*NF+f]
   int* sensors = nullptr;   // [e]
   int* sens_tgt = nullptr;  // sensor resolution scratch [e*2]

@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs a) {
   const bool shared_minv = a.minv_stride == 0;
   // reference tables and the tile's inputs are fetched together (one wait)
   static_assert(MG * Ms <= 256, "face tables fit one pass");
-  VolTableFetch<D, P, PH, true> tf;
+  VolTableFetch<D, P, PH> tf;
   tf.fetch(a.phi, a.dphi, a.phi_w, a.dphi_w, a.Minv, MODE == 1 && shared_minv, tid);
   double psi_r = 0.0, psiw_r = 0.0;
   if (tid < MG * Ms) { psi_r = a.psi[tid]; psiw_r = a.psi_w[tid]; }

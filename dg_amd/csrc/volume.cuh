@@ -45,12 +45,12 @@ struct VolTables {
 template <int D, int P, int PH>
 __device__ inline void load_vol_tables(const VolTables<D, P, PH>& t, const double* phi, const double* dphi,
                                        const double* phi_w, const double* dphi_w, const double* Minv,
-                                       bool uniform_minv, int tid, int nthr = 256, bool with_dw = true) {
+                                       bool uniform_minv, int tid, int nthr = 256) {
   using V = Vol<D, P, PH>;
   for (int k = tid; k < V::NTAB_PHI; k += nthr) t.phi[k] = phi[k];
   for (int k = tid; k < V::NTAB_D; k += nthr) {
     const int i = k / (V::NG * D), r = k % (V::NG * D);
-    if (with_dw) t.dw[r * V::Ns + i] = dphi_w[k];
+    t.dw[r * V::Ns + i] = dphi_w[k];
     if constexpr (V::NNC > 0) t.dphi[k] = dphi[k];
   }
   if constexpr (V::NNC > 0)
@@ -62,13 +62,13 @@ __device__ inline void load_vol_tables(const VolTables<D, P, PH>& t, const doubl
 // The same tables for 256-thread blocks in two steps: fetch() issues every
 // global load into registers and store() writes them to LDS, so that a
 // caller can issue its own loads in between and wait once for all of them.
-template <int D, int P, int PH, bool DW>
+template <int D, int P, int PH>
 struct VolTableFetch {
   using V = Vol<D, P, PH>;
   static constexpr int RP = (V::NTAB_PHI + 255) / 256, RD = (V::NTAB_D + 255) / 256;
   static constexpr int RM = (V::Ns * V::Ns + 255) / 256;
   static constexpr bool NC = V::NNC > 0;
-  double phi[RP], pw[NC ? RP : 1], dw[DW ? RD : 1], dphi[NC ? RD : 1], minv[RM];
+  double phi[RP], pw[NC ? RP : 1], dw[RD], dphi[NC ? RD : 1], minv[RM];
   __device__ inline void fetch(const double* phi_g, const double* dphi_g, const double* phi_w, const double* dphi_w,
                                const double* Minv, bool with_minv, int tid) {
 #pragma unroll
@@ -83,7 +83,7 @@ struct VolTableFetch {
     for (int r = 0; r < RD; ++r) {
       const int k = tid + r * 256;
       if (k < V::NTAB_D) {
-        if constexpr (DW) dw[r] = dphi_w[k];
+        dw[r] = dphi_w[k];
         if constexpr (NC) dphi[r] = dphi_g[k];
       }
     }
@@ -107,7 +107,7 @@ struct VolTableFetch {
       const int k = tid + r * 256;
       if (k < V::NTAB_D) {
         const int i = k / (V::NG * D), q = k % (V::NG * D);
-        if constexpr (DW) t.dw[q * V::Ns + i] = dw[r];
+        t.dw[q * V::Ns + i] = dw[r];
         if constexpr (NC) t.dphi[k] = dphi[r];
       }
     }
