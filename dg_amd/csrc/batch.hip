@@ -129,7 +129,7 @@ __device__ __forceinline__ void batch_segment(const BatchArgs& a, const BatchSeg
 
 // LB: the launch bound, WPE: the waves per SIMD the registers must allow.
 // Bound by issue and latency, not by memory (two state vectors a step): 256
-// two-fluid problems (540k elements, 128 threads): 0.241 ms a step against
+// two-fluid problems (540k elements, 128 threads): 0.238 ms a step against
 // 0.49 ms of the kernel it replaced, 0.197 at 256 threads.
 template <int PH, int FL, int R, int LB, int WPE>
 __global__ __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(WPE))) void k_batch(BatchArgs a) {

@@ -594,7 +594,7 @@ static dgx_status timed_limit(Solver& s, int limiter, double* U, hipStream_t st)
 #ifndef DGX_RK_HR2D
 // 1: on grids where the one-launch HR kernels apply (Solver::hr2d) the RK
 // driver limits out of place with them; 0: the two sweep launches in place.
-// On the 1024x512 p=2 two-fluid grid: 110 us (k_hr2d_rows) against 212 us an
+// On the 1024x512 p=2 two-fluid grid: 94 us (k_hr2d_rows) against 209 us an
 // application.
 #define DGX_RK_HR2D 1
 #endif
