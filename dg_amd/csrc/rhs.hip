@@ -380,7 +380,9 @@ __global__ __launch_bounds__(256) void k_upa_max(const double* __restrict__ U, i
     v = upa<D, PH>(u);
   }
   if (n == 0) partial[gridDim.x] = v;  // node 0, where idamax starts
-  const double m = block_max(v, red);
+  // a lane that brought a NaN into the reduction would keep it and lose the
+  // values that it is handed on the way
+  const double m = block_max(skip_nan_max(0.0, v), red);
   if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
